@@ -1,0 +1,391 @@
+"""Performance cases of the framework: what a serving program has it do.
+
+Each case goes through a public entry point (the linear ops, the drop-in ops,
+the vision step, the language-model step) at the sizes of the Qwen3-VL presets,
+from the single picked row of a prefill's tail to the whole 8B step.
+``listed`` holds the standing cases, ``draw`` makes more of the same ranges.
+"""
+import dataclasses
+import math
+
+import torch
+
+from fastforward_amd import ops, vision
+from fastforward_amd.linear import FP8Linear, Int4, RuntimeScaleLinear
+from fastforward_amd.runtime import PRESETS, Runtime
+from fastforward_amd.synthetic import linear_shapes, make_model, make_request
+
+BF16, F32, F64 = torch.bfloat16, torch.float32, torch.float64
+E4M3 = torch.float8_e4m3fn
+DEVICE = "cuda"
+STATIC_BOUND = 8.0          # calibrated activation bound of the static FP8 linears
+
+
+def listed():
+    return [
+        # the pick-only tail's o projection at the 2B width: one row, the smallest call of the step
+        dict(name="fp8_o_2b_row", kind="fp8", mode="dynamic", m=1, n=2048, k=2048),
+        # the 2B prompt (320 tokens) through the down projection: few tiles, a long k
+        dict(name="fp8_down_2b_320", kind="fp8", mode="dynamic", m=320, n=2048, k=6144),
+        # calibrated (static-scale) FP8 at the deployed 176-token bucket, 8B qkv: weight-bound
+        dict(name="fp8_static_qkv_8b_176", kind="fp8", mode="static", m=176, n=6144, k=4096),
+        # the largest single linear of the benchmark's microbench list: 32B widths, 1024 tokens
+        dict(name="fp8_32b_1024", kind="fp8", mode="dynamic", m=1024, n=25600, k=5120),
+        # W4A16 (symmetric, group 128), the 8B down projection over the 576-token prompt
+        dict(name="int4_down_8b_576", kind="int4", m=576, n=4096, k=12288, group=128, symmetric=True, swiglu=False),
+        # the asymmetric group-32 int4 bank's gate/up with its SwiGLU, 4B widths, deployed bucket
+        dict(name="int4_gateup_4b_176", kind="int4", m=176, n=2 * 9728, k=2560, group=32, symmetric=False,
+             swiglu=True),
+        # causal GQA prefill attention of the 8B step
+        dict(name="attention_8b_576", kind="attention", t=576, heads=32, kv_heads=8),
+        # the same at the 32B head count and a long ragged prompt
+        dict(name="attention_32b_1999", kind="attention", t=1999, heads=64, kv_heads=8),
+        # residual add + RMSNorm with a DeepStack image block, the 8B step's row kernel
+        dict(name="add_rms_8b_576", kind="add_rms", t=576, h=4096, start=4, nv=512),
+        # one block + merger of the 8B vision tower on the deployed 320 x 320 canvas (400 patches)
+        dict(name="vision_block_8b_400", kind="vision", preset="qwen3vl-8b", gh=20, gw=20, depth=1),
+        # the whole 8B vision tower on a 512 x 1024 image (2048 patches), one graph replay
+        dict(name="vision_tower_8b_2048", kind="vision", preset="qwen3vl-8b", gh=32, gw=64, depth=27),
+        # the whole 8B FP8 prefill + choice-score step, one graph replay
+        dict(name="lm_8b_fp8_576", kind="lm", preset="qwen3vl-8b", mode="fp8", tokens=576, gh=16, gw=32),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return min(hi, max(lo, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))))
+
+
+def draw(rng):
+    kind = rng.choice(["fp8", "fp8", "int4", "int4", "attention", "attention", "add_rms", "vision", "vision", "lm"])
+    preset = rng.choice(sorted(PRESETS))
+    cfg = PRESETS[preset]
+    if kind == "fp8":
+        n, k = linear_shapes(cfg)[rng.choice(["qkv", "o", "gateup", "down"])]
+        return dict(kind=kind, mode=rng.choice(["dynamic", "static"]), m=_log_int(rng, 1, 1024), n=n, k=k)
+    if kind == "int4":
+        role = rng.choice(["qkv", "o", "gateup", "down"])
+        n, k = linear_shapes(cfg)[role]
+        symmetric = rng.random() < 0.5
+        return dict(kind=kind, m=_log_int(rng, 1, 1024), n=n, k=k, group=128 if symmetric else 32,
+                    symmetric=symmetric, swiglu=role == "gateup")
+    if kind == "attention":
+        return dict(kind=kind, t=_log_int(rng, 16, 2000), heads=cfg.heads, kv_heads=cfg.kv_heads)
+    if kind == "add_rms":
+        t = _log_int(rng, 1, 2048)
+        nv = rng.randint(0, t)
+        return dict(kind=kind, t=t, h=cfg.hidden, start=rng.randint(0, t - nv), nv=nv)
+    if kind == "vision":
+        vc = vision.VISION_PRESETS[preset]
+        gh = 2 * _log_int(rng, 3, 24)
+        gw = 2 * _log_int(rng, 3, min(24, 1024 // gh))
+        return dict(kind=kind, preset=preset, gh=gh, gw=gw, depth=rng.choice([1, vc.depth]))
+    # the language-model step: the sizes whose whole step costs no more than the listed one
+    preset = rng.choice(["qwen3vl-2b", "qwen3vl-4b", "qwen3vl-8b"])
+    mode = rng.choice(["fp8", "fp8_static", "w4a16"] if preset != "qwen3vl-8b" else ["fp8", "fp8_static"])
+    gh, gw = rng.randint(2, 16), rng.randint(2, 16)
+    tokens = min(576, gh * gw + 4 + _log_int(rng, 20, 320))
+    return dict(kind="lm", preset=preset, mode=mode, tokens=tokens, gh=gh, gw=gw)
+
+
+# ---------------------------------------------------------------- inputs
+
+def _gen(seed, part=0):
+    g = torch.Generator(device=DEVICE)
+    g.manual_seed(seed * 1009 + part)
+    return g
+
+
+def _randn(g, *shape, scale=1.0):
+    return (torch.randn(shape, generator=g, device=DEVICE) * scale).to(BF16)
+
+
+def _linear_inputs(case, seed):
+    # normalised activations with some channels much larger than the rest, as after an RMSNorm
+    g = _gen(seed)
+    w = _randn(g, case["n"], case["k"], scale=0.02)
+    gain = 1 + 4 * (torch.rand(case["k"], generator=g, device=DEVICE) < 0.01)
+    x = (torch.randn((case["m"], case["k"]), generator=g, device=DEVICE) * gain).to(BF16)
+    return w, x
+
+
+def _attention_inputs(case, seed):
+    # q, k as qk_pair leaves them (unit RMS heads); v the strided view of a packed qkv product
+    t, hq, hk, d = case["t"], case["heads"], case["kv_heads"], 128
+    g = _gen(seed)
+    q = _randn(g, 1, hq, t, d)
+    k = _randn(g, 1, hk, t, d)
+    qkv = _randn(g, 1, t, (hq + 2 * hk) * d)
+    v = qkv[..., (hq + hk) * d:].view(1, t, hk, d).transpose(1, 2)
+    return q, k, v
+
+
+def _add_rms_inputs(case, seed):
+    t, h, nv = case["t"], case["h"], case["nv"]
+    g = _gen(seed)
+    a, b = _randn(g, 1, t, h, scale=2.0), _randn(g, 1, t, h)
+    deep = _randn(g, nv, h) if nv else None
+    w = (1 + 0.1 * torch.randn(h, generator=g, device=DEVICE)).to(BF16)
+    return a, b, deep, w
+
+
+def _vision_config(case):
+    vc = vision.VISION_PRESETS[case["preset"]]
+    if case["depth"] == vc.depth:
+        return vc
+    return dataclasses.replace(vc, depth=case["depth"], deepstack=())
+
+
+def _vision_inputs(case, seed):
+    """Raw tower weights (unpadded) and an image of smooth gradients with noise."""
+    vc = _vision_config(case)
+    g = _gen(seed)
+    H, W4 = vc.hidden, vc.hidden * vc.merge ** 2
+    lin = lambda n, k: (_randn(g, n, k, scale=0.02), _randn(g, n, scale=0.02))  # noqa: E731
+    norm = lambda n: ((1 + 0.1 * torch.randn(n, generator=g, device=DEVICE)).to(BF16),  # noqa: E731
+                      _randn(g, n, scale=0.1))
+    raw = dict(patch=lin(H, 1536), pos=_randn(g, vc.pos_side ** 2, H, scale=0.02), blocks=[], deep=[])
+    for _ in range(vc.depth):
+        raw["blocks"].append(dict(norm1=norm(H), qkv=lin(3 * H, H), proj=lin(H, H), norm2=norm(H),
+                                  fc1=lin(vc.inter, H), fc2=lin(H, vc.inter)))
+    merger = lambda post: dict(norm=norm(W4 if post else H), fc1=lin(W4, W4),  # noqa: E731
+                               fc2=lin(vc.out_hidden, W4))
+    raw["merger"] = merger(False)
+    raw["deep"] = [merger(True) for _ in vc.deepstack]
+    hgt, wid = 16 * case["gh"], 16 * case["gw"]
+    y = torch.arange(hgt, device=DEVICE, dtype=F32)[:, None, None]
+    x = torch.arange(wid, device=DEVICE, dtype=F32)[None, :, None]
+    c = torch.arange(3, device=DEVICE, dtype=F32)[None, None, :]
+    smooth = 127 + 80 * torch.sin(y / 40 + c) * torch.cos(x / 55 - c)
+    noise = 15 * torch.randn((hgt, wid, 3), generator=g, device=DEVICE)
+    return vc, raw, (smooth + noise).clamp(0, 255).to(torch.uint8)
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "fp8":
+        w, x = _linear_inputs(case, seed)
+        op = FP8Linear(w) if case["mode"] == "dynamic" else RuntimeScaleLinear(w, 448.0 / STATIC_BOUND)
+        return dict(kind=kind, op=op, x=x)
+    if kind == "int4":
+        w, x = _linear_inputs(case, seed)
+        return dict(kind=kind, op=Int4(w, group=case["group"], symmetric=case["symmetric"]).pack(), x=x,
+                    swiglu=case["swiglu"])
+    if kind == "attention":
+        q, k, v = _attention_inputs(case, seed)
+        return dict(kind=kind, q=q, k=k, v=v, scale=128 ** -0.5)
+    if kind == "add_rms":
+        a, b, deep, w = _add_rms_inputs(case, seed)
+        return dict(kind=kind, a=a, b=b, deep=deep, module=ops.RMSNorm(w), start=case["start"], nv=case["nv"])
+    if kind == "vision":
+        vc, raw, rgb = _vision_inputs(case, seed)
+        lin, norm = (lambda p: vision.Lin(*p)), (lambda p: vision.Norm(*p))
+        blocks = []
+        for r in raw["blocks"]:
+            w1, b1, w2 = vision.pad_mlp(vc, *r["fc1"], r["fc2"][0])
+            blocks.append(vision.VBlock(norm(r["norm1"]), lin(r["qkv"]), lin(r["proj"]), norm(r["norm2"]),
+                                        vision.Lin(w1, b1), vision.Lin(w2, r["fc2"][1])))
+        mg = lambda r, post: vision.VMerger(norm(r["norm"]), lin(r["fc1"]), lin(r["fc2"]), post)  # noqa: E731
+        weights = vision.VisionWeights(lin(raw["patch"]), raw["pos"], blocks, mg(raw["merger"], False),
+                                       [mg(r, True) for r in raw["deep"]])
+        rt = vision.VisionRuntime(vc, weights, case["gh"], case["gw"])
+        rt.set_image(rgb)
+        rt.capture()
+        return dict(kind=kind, rt=rt)
+    cfg = PRESETS[case["preset"]]
+    weights = make_model(cfg, mode=case["mode"], seed=seed, static_bound=STATIC_BOUND)
+    rt = Runtime(cfg, weights, case["tokens"])
+    rt.set_inputs(*make_request(cfg, case["tokens"], case["gh"], case["gw"], seed=seed))
+    rt.capture()
+    return dict(kind="lm", rt=rt)
+
+
+def run(state):
+    kind = state["kind"]
+    if kind == "fp8":
+        return state["op"](state["x"])
+    if kind == "int4":
+        return state["op"].swiglu(state["x"]) if state["swiglu"] else state["op"](state["x"])
+    if kind == "attention":
+        return ops.attention_direct(state["q"], state["k"], state["v"], state["scale"])
+    if kind == "add_rms":
+        return ops.add_rms(state["a"], state["b"], state["deep"], state["module"], state["start"], state["nv"])
+    if kind == "vision":
+        merged, deep = state["rt"].replay()
+        return [merged, *deep]
+    return state["rt"].replay()
+
+
+# ---------------------------------------------------------------- work
+
+def _lm_work(case):
+    cfg, t = PRESETS[case["preset"]], case["tokens"]
+    shapes = linear_shapes(cfg)
+    wbytes = 0.5 if case["mode"] == "w4a16" else 1.0
+    full = cfg.layers - 1
+    flops, weights = 0.0, 0.0
+    for role, (n, k) in shapes.items():
+        rows = t * full + (t if role == "qkv" else 1)      # the last layer scores the picked row only
+        flops += 2.0 * rows * n * k
+        weights += cfg.layers * n * k * wbytes
+    flops += full * 4.0 * cfg.heads * cfg.head_dim * t * (t + 1) / 2
+    return dict(bytes=weights + 4.0 * t * cfg.hidden, flops=flops)
+
+
+def _vision_work(case):
+    vc, n = _vision_config(case), case["gh"] * case["gw"]
+    H, I, W4 = vc.hidden, vc.inter, vc.hidden * vc.merge ** 2
+    nm, mergers = n // vc.merge ** 2, len(vc.deepstack) + 1
+    weights = 1536 * H + vc.depth * H * (4 * H + 2 * I) + mergers * W4 * (W4 + vc.out_hidden)
+    flops = 2.0 * n * 1536 * H + vc.depth * (2.0 * n * H * (4 * H + 2 * I) + 4.0 * n * n * H)
+    flops += mergers * 2.0 * nm * W4 * (W4 + vc.out_hidden)
+    return dict(bytes=2.0 * weights + 768.0 * n + mergers * 2.0 * nm * vc.out_hidden, flops=flops)
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "fp8":
+        m, n, k = case["m"], case["n"], case["k"]
+        return dict(bytes=2.0 * m * k + n * k + 4.0 * n + 2.0 * m * n, flops=2.0 * m * n * k)
+    if kind == "int4":
+        m, n, k = case["m"], case["n"], case["k"]
+        out = n // 2 if case["swiglu"] else n
+        return dict(bytes=2.0 * m * k + n * k / 2 + 4.0 * n * k / case["group"] + 2.0 * m * out,
+                    flops=2.0 * m * n * k)
+    if kind == "attention":
+        t, hq, hk = case["t"], case["heads"], case["kv_heads"]
+        return dict(bytes=2.0 * t * 128 * (2 * hq + 2 * hk), flops=4.0 * hq * 128 * t * (t + 1) / 2)
+    if kind == "add_rms":
+        t, h, nv = case["t"], case["h"], case["nv"]
+        return dict(bytes=2.0 * h * (4 * t + nv + 1), flops=5.0 * t * h)
+    return _vision_work(case) if kind == "vision" else _lm_work(case)
+
+
+# ---------------------------------------------------------------- references
+
+def tolerance(case):
+    """About four times the distance of the present results from ``exact``."""
+    kind = case["kind"]
+    if kind == "fp8":
+        return {"rel": 1.6e-2}                              # 1.7e-3 (static) to 4.6e-3 (dynamic: 13-bit block sums)
+    if kind == "int4":
+        return {"rel": 1.6e-2 if case["swiglu"] else 8e-3}  # 4.2e-3 and 2.2e-3
+    if kind == "attention":
+        return {"rel": 8e-3}                                # 2.0e-3
+    if kind == "add_rms":
+        return {"rel": 1.2e-2}                              # 3.3e-3
+    if kind == "vision":
+        return {"rel": 2.5e-2 if case["depth"] == 1 else 5e-2}  # 6.3e-3 and 1.3e-2
+    # Two orders of the k sums (o and down in one and in two parts) put the logits of the 8B step
+    # 0.12 to 0.39 apart: the random-init step is chaotic in its e4m3 requantisations.
+    return {"rel": 0.9}
+
+
+def _div(a, b):
+    """a / b rounded once to fp32 (a scalar divisor is a reciprocal product in torch's GPU kernel)."""
+    return (a.to(F64) / b).to(F32)
+
+
+def _exact_fp8(case, seed):
+    w, x = _linear_inputs(case, seed)
+    wf, xf = w.to(F32), x.to(F32)
+    if case["mode"] == "dynamic":       # one scale per weight row, one per token
+        sw = _div(wf.abs().amax(1, keepdim=True).clamp_min(1e-12), 448)
+        sx = _div(xf.abs().amax(1, keepdim=True).clamp_min(1e-12), 448)
+        qx = _div(xf, sx).clamp(-448, 448).to(E4M3)
+    else:                               # one scale per tensor, the calibrated activation multiplier
+        sw = _div(wf.abs().max().reshape(1, 1), 448)
+        sx = torch.tensor([[STATIC_BOUND / 448.0]], device=DEVICE)
+        qx = (xf * (448.0 / STATIC_BOUND)).clamp(-448, 448).to(E4M3)
+    qw = _div(wf, sw).clamp(-448, 448).to(E4M3)
+    return (qx.to(F64) @ qw.to(F64).T) * sx.to(F64) * sw.to(F64).reshape(1, -1)
+
+
+def _exact_int4(case, seed):
+    w, x = _linear_inputs(case, seed)
+    n, k = w.shape
+    v = w.to(F32).reshape(n, -1, case["group"])
+    if case["symmetric"]:
+        s = _div(v.abs().amax(-1, keepdim=True).clamp_min(1e-6), 7).to(BF16).to(F32)
+        z = torch.zeros_like(s)
+        q = (_div(v, s).round() + 8).clamp(0, 15)
+    else:
+        low, high = v.amin(-1, keepdim=True), v.amax(-1, keepdim=True)
+        s = _div(high - low, 15).clamp_min(1e-6)
+        q = _div(v - low, s).round().clamp(0, 15)
+        s, z = s.to(BF16), (low + 8 * s).to(BF16)
+    dq = ((q.to(F64) - 8) * s.to(F64) + z.to(F64)).reshape(n, k)
+    y = x.to(F64) @ dq.T
+    if not case["swiglu"]:
+        return y
+    gate, up = y.chunk(2, -1)
+    return gate / (1 + torch.exp(-gate)) * up
+
+
+def _exact_attention(case, seed):
+    q, k, v = _attention_inputs(case, seed)
+    t, rep = case["t"], case["heads"] // case["kv_heads"]
+    mask = torch.ones(t, t, dtype=torch.bool, device=DEVICE).triu(1)
+    out = torch.empty((1, t, case["heads"], 128), dtype=F64, device=DEVICE)
+    for h in range(case["heads"]):
+        s = q[0, h].to(F64) @ k[0, h // rep].to(F64).T * 128 ** -0.5
+        out[0, :, h] = torch.softmax(s.masked_fill(mask, -math.inf), -1) @ v[0, h // rep].to(F64)
+    return out
+
+
+def _exact_add_rms(case, seed):
+    a, b, deep, w = _add_rms_inputs(case, seed)
+    x = a.to(F64) + b.to(F64)
+    if deep is not None:
+        x[0, case["start"]:case["start"] + case["nv"]] += deep.to(F64)
+    return x, x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * w.to(F64)
+
+
+def _exact_vision(case, seed):
+    vc, raw, rgb = _vision_inputs(case, seed)
+    gh, gw, H = case["gh"], case["gw"], vc.hidden
+    hd, n = H // vc.heads, gh * gw
+    lin = lambda x, p: x @ p[0].to(F64).T + p[1].to(F64)  # noqa: E731
+    norm = lambda x, p: torch.nn.functional.layer_norm(x, x.shape[-1:], p[0].to(F64), p[1].to(F64), vc.eps)  # noqa: E731
+    order = lambda x: x.reshape(gh // 2, 2, gw // 2, 2, -1).transpose(1, 2).reshape(n, -1)  # noqa: E731
+    # patches (channel, frame, y, x) in 2 x 2 merge order, both frames the same image
+    px = ((rgb.to(F64) - 127.5) / 127.5).reshape(gh, 16, gw, 16, 3).permute(0, 2, 4, 1, 3).reshape(gh, gw, 3, 1, 256)
+    h = lin(order(px.expand(-1, -1, -1, 2, -1).reshape(gh, gw, -1)), raw["patch"])
+    # bilinear (align-corners) position embedding
+    grid = raw["pos"].to(F64).reshape(vc.pos_side, vc.pos_side, H).permute(2, 0, 1)[None]
+    pos = torch.nn.functional.interpolate(grid, size=(gh, gw), mode="bilinear", align_corners=True)
+    h = h + order(pos[0].permute(1, 2, 0))
+    # 2-D rotary angles: a quarter of the head's pairs by row, a quarter by column
+    inv = 1.0 / vc.theta ** (torch.arange(0, hd // 2, 2, device=DEVICE, dtype=F64) / (hd // 2))
+    r = torch.arange(gh, device=DEVICE, dtype=F64)[:, None, None].expand(gh, gw, 1) * inv
+    c = torch.arange(gw, device=DEVICE, dtype=F64)[None, :, None].expand(gh, gw, 1) * inv
+    f = order(torch.cat([r, c], -1))
+    cos, sin = torch.cat([f, f], -1).cos()[:, None], torch.cat([f, f], -1).sin()[:, None]
+    rot = lambda x: x * cos + torch.cat([-x[..., hd // 2:], x[..., :hd // 2]], -1) * sin  # noqa: E731
+
+    def merge(m, post):
+        x = norm(h.reshape(n // 4, 4 * H), m["norm"]) if post else norm(h, m["norm"]).reshape(n // 4, 4 * H)
+        return lin(torch.nn.functional.gelu(lin(x, m["fc1"])), m["fc2"])
+
+    deep = []
+    for j, blk in enumerate(raw["blocks"]):
+        q, k, v = lin(norm(h, blk["norm1"]), blk["qkv"]).reshape(n, 3, vc.heads, hd).unbind(1)
+        q, k = rot(q), rot(k)
+        z = torch.empty((n, vc.heads, hd), dtype=F64, device=DEVICE)
+        for i in range(vc.heads):
+            z[:, i] = torch.softmax(q[:, i] @ k[:, i].T * hd ** -0.5, -1) @ v[:, i]
+        h = h + lin(z.reshape(n, H), blk["proj"])
+        u = lin(norm(h, blk["norm2"]), blk["fc1"])
+        h = h + lin(torch.nn.functional.gelu(u, approximate="tanh"), blk["fc2"])
+        if j in vc.deepstack:
+            deep.append(merge(raw["deep"][vc.deepstack.index(j)], True))
+    return [merge(raw["merger"], False), *deep]
+
+
+def exact(case, seed):
+    """64-bit results. The language-model step has none: its e4m3 requantisations
+    turn a last-bit difference of any layer into other codes of the next."""
+    kind = case["kind"]
+    if kind == "lm":
+        return None
+    return {"fp8": _exact_fp8, "int4": _exact_int4, "attention": _exact_attention, "add_rms": _exact_add_rms,
+            "vision": _exact_vision}[kind](case, seed)
