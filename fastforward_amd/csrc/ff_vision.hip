@@ -171,19 +171,34 @@ __global__ __launch_bounds__(kThreads) void layer_norm_kernel(const bf16_t* __re
 // ---------------------------------------------------------------- bf16 GEMM
 //
 // y[m, n] = epilogue(sum_k a[m, k] w[n, k]) with a (M, K) and w (N, K) bf16,
-// both K-contiguous (torch Linear weights). A workgroup of 4 waves (2 x 2)
-// owns a BM x BN tile; each wave (BM/2) x (BN/2) as 16 x 16 tiles of
-// v_mfma_f32_16x16x32_bf16. K advances 64 elements (128 bytes) per stage:
-// both operands go global -> LDS with global_load_lds_dwordx4 (8 rows x 128 B
-// per instruction, XOR-swizzled 16-byte chunks), S stages with S - 1 in
-// flight, one barrier per stage. Lane l (row l % 16, g = l / 16) reads chunks
-// 2g and 2g + 1 of its row for the two MFMAs of a stage: k [16 g, 16 g + 8)
-// and [16 g + 8, 16 g + 16) of the 64, the same k for A and B.
+// both K-contiguous (torch Linear weights). A workgroup of 4 waves (2 x 2) owns
+// a 32 WI x 32 WJ tile; each wave WI x WJ tiles of v_mfma_f32_16x16x32_bf16. K
+// advances 64 elements (128 bytes) per stage: both operands go global -> LDS
+// with global_load_lds_dwordx4 (8 rows x 128 B per instruction), S stages deep.
+// Chunk c of row r sits at slot c ^ (r % 8) ^ (r / 8 % 2). Lane l (row l % 16,
+// g = l / 16) reads chunks 2g and 2g + 1 of its row for the two MFMAs of a
+// stage: k [16 g, 16 g + 8) and [16 g + 8, 16 g + 16) of the 64, the same k for
+// A and B, and the same order at every tile, so every tile gives the same bits.
+//
+// What bounds it: the operands' way from L2 into LDS (a work-skipping copy of
+// the 2048 x 4352 x 1152 launch: 18 us for the copies alone, 20 us for the
+// MFMAs alone, 24 us for both), which is why the tile is as large as one round
+// of the grid allows, and about 10 us per launch outside the main loop (first
+// stage, tile stores). Inside a stage the two MFMA groups are software-pipelined:
+// the second group's fragments are read from LDS under the first group's MFMAs
+// and the next stage's first fragments under the second group's, with the
+// stage's one wait and barrier between the groups, where the reads that the
+// barrier has to cover are already done. The stage just consumed is refilled by
+// DMAs spread over the second group.
+// 2048 rows, weights streamed, against the previous two-barrier-free 128 x 128
+// and 64 x 128 tiles at two and three workgroups per CU (same bits): fc1 with
+// GELU 46.9 -> 28.5 us, qkv 26.5 -> 21.6, fc2 40.2 -> 36.0, proj 14.4 -> 13.2; at
+// 400 rows qkv 12.6 -> 10.0, fc1 18.0 -> 12.3.
 //
 // Epilogue (the bf16 module boundaries of the reference): v = bf16(acc + bias);
 // kGeluTanh: v = bf16(gelu_tanh(v)); kGeluErf: v = bf16(gelu(v)); with a
-// residual r: y = bf16(r + v) (r may be y itself: each element is read and
-// written by one thread).
+// residual r: y = bf16(r + v) (r may be y itself: a workgroup reads and writes
+// its own tile only).
 constexpr int kActNone = 0, kGeluTanh = 1, kGeluErf = 2;
 
 __device__ __forceinline__ f32x4 mfma_bf16(const u32x4& a, const u32x4& b, const f32x4& c) {
@@ -191,120 +206,222 @@ __device__ __forceinline__ f32x4 mfma_bf16(const u32x4& a, const u32x4& b, const
                                                  c, 0, 0, 0);
 }
 
-// GELU with the tanh approximation, as torch computes it in fp32 for bf16
-// tensors: 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))).
+// GELU with the tanh approximation, 0.5 x (1 + tanh(u)) with u = sqrt(2/pi) (x +
+// 0.044715 x^3), evaluated as x / (1 + exp(-2u)), which is the same function:
+// one hardware exp2 and one reciprocal (1 ulp each) instead of tanhf's two
+// branches, and no cancellation in 1 + tanh(u) for negative x.
 __device__ __forceinline__ float gelu_tanh(float x) {
-  const float k_beta = 0.7978845608028654f;  // sqrt(2 / pi)
-  const float inner = k_beta * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (1.0f + tanhf(inner));
+  constexpr float c1 = -2.3022081997f;   // -2 sqrt(2/pi) log2(e)
+  constexpr float c3 = -0.10294324080f;  // 0.044715 c1
+  const float u = x * __builtin_fmaf(c3, x * x, c1);
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(u));
 }
 
 // Exact GELU: x / 2 (1 + erf(x / sqrt 2)).
 __device__ __forceinline__ float gelu_erf(float x) { return x * 0.5f * (1.0f + erff(x * 0.7071067811865476f)); }
 
-template <int BM, int BN, int S>
-struct GemmCfg {
-  static constexpr int RA = BM / 16, RB = BN / 16;
-  static constexpr int BLOCKS = 2 * (RA + RB);  // 1 KB blocks per stage
-  static constexpr int STAGE = BLOCKS * 1024;
-  static constexpr int WI = RA / 2, WJ = RB / 2;
-  static constexpr int SMEM = S * STAGE;
-  static_assert(SMEM <= 160 * 1024, "LDS budget");
-  static_assert(RA % 2 == 0 && RB % 2 == 0 && BLOCKS % 4 == 0, "2 x 2 waves");
+template <int WI, int WJ>
+struct PipeCfg {
+  static constexpr int BM = 32 * WI, BN = 32 * WJ;
+  static constexpr int STAGE = (BM + BN) * 128;  // one 64-k stage of both operands
+  static constexpr int PW = WI + WJ;             // 1 KB DMAs per wave and stage
 };
 
-template <int BM, int BN, int S, int OCC, int ACT, bool RESID>
-__global__ __launch_bounds__(kThreads, OCC) void gemm_bf16_kernel(
+// s_waitcnt vmcnt(n * PW + X) for the run-time n in [0, N].
+template <int N, int PW, int X>
+__device__ __forceinline__ void wait_stages(int n) {
+  if constexpr (N == 0) {
+    wait_vmcnt<X>();
+  } else {
+    if (n >= N) wait_vmcnt<N * PW + X>();
+    else wait_stages<N - 1, PW, X>(n);
+  }
+}
+
+__device__ __forceinline__ void mfma_bf16_acc(f32x4& acc, const i32x4v& a, const i32x4v& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+
+template <int WI, int WJ, int S, int ACT, bool RESID>
+__global__ __launch_bounds__(kThreads, 1) void gemm_bf16_kernel(
     const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
-    bf16_t* y, int64_t ldy, const bf16_t* resid, int64_t ldr, int M, int N, int K, int tiles_m, int tiles_n) {
-  using C = GemmCfg<BM, BN, S>;
-  __shared__ __align__(1024) uint8_t smem[C::SMEM];
-  __shared__ __align__(16) bf16_t sbias[BN];  // the tile's bias columns
-  static_assert(BN == 128, "one wave's dword DMA carries the tile's bias");
-  const int nblk = tiles_m * tiles_n;
-  const int blk_id = blockIdx.x;
-  int logical = blk_id;
-  if (nblk % kXcds == 0) logical = (blk_id % kXcds) * (nblk / kXcds) + blk_id / kXcds;
-  const int tm = logical % tiles_m, tn = logical / tiles_m;  // M fastest: an XCD's tiles share weight slabs
+    bf16_t* y, int64_t ldy, const bf16_t* resid, int64_t ldr, int M, int N, int K, int tiles_m, int tiles_n,
+    int strips) {
+  using C = PipeCfg<WI, WJ>;
+  constexpr int BM = C::BM, BN = C::BN, PW = C::PW;
+  constexpr int RQ = RESID ? WI * WJ / 2 : 0;  // 1 KB residual DMAs per wave
+  static_assert(!RESID || WI * WJ % 2 == 0, "whole DMA instructions per residual slab");
+  constexpr int RES = RESID ? BM * BN * 2 : 0;
+  static_assert(S * C::STAGE + RES + 1024 <= 160 * 1024, "LDS budget");
+  __shared__ __align__(1024) uint8_t smem[S * C::STAGE + RES];
+  __shared__ __align__(16) bf16_t sbias[256];
+
+  // XCD x (workgroups b with b % 8 == x) takes one contiguous run of the tile
+  // sequence, which walks strips of rps tile rows, rows fastest inside a strip:
+  // its tiles then read a strip of the activations and a slab of the weights,
+  // and each XCD's L2 fetches those once.
+  const int nblk = tiles_m * tiles_n, xcd = blockIdx.x % kXcds;
+  const int seq = xcd * (nblk / kXcds) + min(xcd, nblk % kXcds) + blockIdx.x / kXcds;
+  const int rps = (tiles_m + strips - 1) / strips;
+  const int strip = seq / (rps * tiles_n);
+  const int in = seq - strip * rps * tiles_n, rows = min(rps, tiles_m - strip * rps);
+  const int tm = strip * rps + in % rows, tn = in / rows;
   const int m0 = tm * BM, n0 = tn * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int r16 = lane & 15, g = lane >> 4;
+  const int nk = K / 64;
 
-  // Sources of this lane for each 1 KB block it loads (k offset 0); rows past
+  // Sources of this lane for the 1 KB blocks it loads (k offset 0); rows past
   // M / N are clamped (in bounds; masked at the store).
-  constexpr int PER_WAVE = C::BLOCKS / 4;
-  const uint8_t* src[PER_WAVE];
+  const uint8_t* src[PW];
 #pragma unroll
-  for (int i = 0; i < PER_WAVE; ++i) {
-    const int blk = wave + 4 * i, h = blk & 1;
-    const int rr = 8 * h + (lane >> 3);
-    const int ch = (lane & 7) ^ (rr >> 1);
-    if (blk < 2 * C::RA) {
+  for (int i = 0; i < PW; ++i) {
+    const int blk = wave + 4 * i;
+    const int rr = 8 * (blk & 1) + (lane >> 3);
+    const int ch = (lane & 7) ^ (rr & 7) ^ (rr >> 3);
+    if (blk < 4 * WI) {
       const int row = min(m0 + (blk >> 1) * 16 + rr, M - 1);
       src[i] = reinterpret_cast<const uint8_t*>(a + (int64_t)row * lda) + 16 * ch;
     } else {
-      const int row = min(n0 + ((blk - 2 * C::RA) >> 1) * 16 + rr, N - 1);
+      const int row = min(n0 + ((blk - 4 * WI) >> 1) * 16 + rr, N - 1);
       src[i] = reinterpret_cast<const uint8_t*>(w + (int64_t)row * K) + 16 * ch;
     }
   }
-  const uint32_t lds0 = lds_addr(smem) + (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 1024;
-  auto issue = [&](int kt, int buf) {
-#pragma unroll
-    for (int i = 0; i < PER_WAVE; ++i) lds_dma16(src[i] + (int64_t)kt * 128, lds0 + buf * C::STAGE + 4 * i * 1024);
-  };
+  const uint32_t lds0 = lds_addr(smem) + (uint32_t)wave * 1024;
+  auto issue1 = [&](int i, int kt, uint32_t buf) { lds_dma16(src[i] + (int64_t)kt * 128, lds0 + buf + 4096u * i); };
 
-  f32x4 acc[C::WI][C::WJ];
+  f32x4 acc[WI][WJ];
 #pragma unroll
-  for (int i = 0; i < C::WI; ++i)
+  for (int i = 0; i < WI; ++i)
 #pragma unroll
-    for (int j = 0; j < C::WJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < WJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int KT = K / 64;
-  // Wave 0 copies the tile's bias into LDS ahead of the first stage (one
-  // dword DMA: two columns a lane, the address clamped in bounds past N);
-  // issued before the stages, it has landed when the loop's first wait for
-  // stage 0 returns, and that iteration's barrier publishes it.
-  if (wave == 0) lds_dma4(bias + min(n0 + 2 * lane, N - 2), lds_addr(sbias));
+  // Wave 0 copies the tile's bias into LDS ahead of the stages (two columns a
+  // lane, the address clamped in bounds past N): it has landed when the wait for
+  // stage 0 returns, and the barrier after that publishes it.
+  if (wave == 0) {
 #pragma unroll
-  for (int st = 0; st < S - 1; ++st)
-    if (st < KT) issue(st, st);
-  const int frag = 128 * (r16 & 7) + 1024 * (r16 >> 3);
-  const int c0 = 16 * ((2 * g) ^ (r16 >> 1)), c1 = 16 * ((2 * g + 1) ^ (r16 >> 1));
-  for (int kt = 0; kt < KT; ++kt) {
-    if (kt + S - 2 < KT) wait_vmcnt<(S - 2) * PER_WAVE>();
-    else wait_vmcnt<0>();
-    barrier_lds();  // every wave's loads for stage kt landed; stage kt - 1 fully consumed
-    if (kt + S - 1 < KT) issue(kt + S - 1, (kt + S - 1) % S);
-    const uint8_t* st = smem + (kt % S) * C::STAGE + frag;
-    u32x4 a0[C::WI], a1[C::WI];
-#pragma unroll
-    for (int i = 0; i < C::WI; ++i) {
-      const uint8_t* p = st + 2 * (wm * C::WI + i) * 1024;
-      a0[i] = *reinterpret_cast<const u32x4*>(p + c0);
-      a1[i] = *reinterpret_cast<const u32x4*>(p + c1);
-    }
-#pragma unroll
-    for (int j = 0; j < C::WJ; ++j) {
-      const uint8_t* p = st + (2 * C::RA + 2 * (wn * C::WJ + j)) * 1024;
-      const u32x4 b0 = *reinterpret_cast<const u32x4*>(p + c0);
-      const u32x4 b1 = *reinterpret_cast<const u32x4*>(p + c1);
-#pragma unroll
-      for (int i = 0; i < C::WI; ++i) acc[i][j] = mfma_bf16(b1, a1[i], mfma_bf16(b0, a0[i], acc[i][j]));
-    }
+    for (int q = 0; q < (BN + 127) / 128; ++q)
+      lds_dma4(bias + min(n0 + 128 * q + 2 * lane, N - 2), lds_addr(sbias) + 256u * q);
   }
+#pragma unroll
+  for (int st = 0; st < S; ++st)
+    if (st < nk) {
+#pragma unroll
+      for (int i = 0; i < PW; ++i) issue1(i, st, st * C::STAGE);
+    }
+  // The residual tile, each wave's part on its own, is copied into LDS by 16-byte
+  // DMAs issued when the last stage has been (rows that are not 16-byte aligned
+  // are read from global memory in the epilogue instead).
+  const bool rdma = RESID && ((uintptr_t)resid & 15) == 0 && (ldr & 7) == 0 && (N & 7) == 0;
+  auto issue_resid = [&]() {
+    if constexpr (RESID) {
+      const uint32_t slab = lds_addr(smem) + S * C::STAGE + (uint32_t)wave * (RQ * 1024);
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) {
+        const int c = 64 * q + lane, row = c / (2 * WJ), ch = c % (2 * WJ);
+        const int m = min(m0 + wm * 16 * WI + row, M - 1), n = min(n0 + wn * 16 * WJ + 8 * ch, N - 8);
+        lds_dma16(resid + (int64_t)m * ldr + n, slab + 1024u * q);
+      }
+    }
+  };
+  if (rdma && nk < S) issue_resid();
 
-  // The weight fragment is the MFMA's first operand, so lane (r16, g) of tile
-  // (i, j) holds row m0 + wm BM/2 + 16 i + r16, columns n0 + wn BN/2 + 16 j + 4 g .. + 3.
+  // This lane's piece of row group f of a stage for MFMA group `sub`: chunk 2 g + sub.
+  const int fr = 1024 * (r16 >> 3) + 128 * (r16 & 7), sw = (r16 & 7) ^ (r16 >> 3);
+  const int offA[2] = {fr + 16 * ((2 * g) ^ sw) + wm * WI * 2048, fr + 16 * ((2 * g + 1) ^ sw) + wm * WI * 2048};
+  const int offB[2] = {fr + 16 * ((2 * g) ^ sw) + (2 * WI + wn * WJ) * 2048,
+                       fr + 16 * ((2 * g + 1) ^ sw) + (2 * WI + wn * WJ) * 2048};
+  i32x4v fa[2][WI], fb[2][WJ];
+  auto read1 = [&](int q, const uint8_t* st, auto SUB_) {
+    constexpr int sub = decltype(SUB_)::value;
+    // in the order the MFMAs take them: b0, a0 .. a(WI-1), b1 ..
+    if (q == 0) fb[sub][0] = *reinterpret_cast<const i32x4v*>(st + offB[sub]);
+    else if (q <= WI) fa[sub][q - 1] = *reinterpret_cast<const i32x4v*>(st + offA[sub] + (q - 1) * 2048);
+    else fb[sub][q - WI] = *reinterpret_cast<const i32x4v*>(st + offB[sub] + (q - WI) * 2048);
+  };
+  // The MFMA is issued from inline asm with the accumulator tied; the wait states
+  // that the compiler then does not see (zeroed accumulators before the first
+  // MFMA, the last MFMA before the epilogue reads) are the s_nops here and below.
 #pragma unroll
-  for (int i = 0; i < C::WI; ++i) {
-    const int m = m0 + wm * (BM / 2) + 16 * i + r16;
-    if (m >= M) continue;
+  for (int i = 0; i < WI; ++i)
 #pragma unroll
-    for (int j = 0; j < C::WJ; ++j) {
-      const int n = n0 + wn * (BN / 2) + 16 * j + 4 * g;
-      if (n >= N) continue;  // N % 4 == 0: a 4-column group is all in or all out
-      const u32x2 bb = *reinterpret_cast<const u32x2*>(sbias + n - n0);
+    for (int j = 0; j < WJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+a"(acc[WI - 1][WJ - 1]));
+
+  wait_stages<S - 1, PW, 0>(min(S, nk) - 1);
+  barrier_lds();
+#pragma unroll
+  for (int q = 0; q < WI + WJ; ++q) read1(q, smem, std::integral_constant<int, 0>{});
+
+  // NR fragment reads spread over the first two thirds of a group's NM MFMAs.
+  constexpr int NM = WI * WJ, NR = WI + WJ;
+  constexpr int RSTEP = NM * 2 / 3 / NR > 0 ? NM * 2 / 3 / NR : 1;
+  constexpr int SLOTS = NM * 2 / 3 / RSTEP > 0 ? NM * 2 / 3 / RSTEP : 1;
+  constexpr int RPER = (NR + SLOTS - 1) / SLOTS;
+  uint32_t cur = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    const uint8_t* st = smem + cur;
+    const uint32_t nxt = cur + C::STAGE == S * C::STAGE ? 0u : cur + C::STAGE;
+    const uint8_t* stn = smem + nxt;
+    static_for<0, NM>([&](auto I_) {
+      constexpr int m = decltype(I_)::value, j = m / WI, i = m % WI;
+      mfma_bf16_acc(acc[i][j], fb[0][j], fa[0][i]);
+      if constexpr (m % RSTEP == 0) {
+#pragma unroll
+        for (int p = 0; p < RPER; ++p)
+          if (m / RSTEP * RPER + p < NR) read1(m / RSTEP * RPER + p, st, std::integral_constant<int, 1>{});
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    // stage kt + 1 has landed: later stages (at most S - 2) may stay in flight
+    const int rem = nk - 1 - kt;
+    if (rem > 0) {
+      if (rdma && kt + S - 1 >= nk) wait_stages<(S > 2 ? S - 2 : 0), PW, RQ>(min(S - 1, rem) - 1);
+      else wait_stages<(S > 2 ? S - 2 : 0), PW, 0>(min(S - 1, rem) - 1);
+    }
+    barrier_lds();  // and every wave's reads of stage kt are done
+    const bool more = kt + S < nk;
+    if (rdma && kt + S == nk) issue_resid();
+    static_for<0, NM>([&](auto I_) {
+      constexpr int m = decltype(I_)::value, j = m / WI, i = m % WI;
+      mfma_bf16_acc(acc[i][j], fb[1][j], fa[1][i]);
+      if constexpr (m % RSTEP == 0) {
+#pragma unroll
+        for (int p = 0; p < RPER; ++p)
+          if (m / RSTEP * RPER + p < NR) read1(m / RSTEP * RPER + p, stn, std::integral_constant<int, 0>{});
+      }
+      if (more) {
+#pragma unroll
+        for (int d = m * PW / NM; d < (m + 1) * PW / NM; ++d) issue1(d, kt + S, cur);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    cur = nxt;
+  }
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+a"(acc[WI - 1][WJ - 1]));
+#pragma unroll
+  for (int i = 0; i < WI; ++i)
+#pragma unroll
+    for (int j = 0; j < WJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+
+  if constexpr (RESID) wait_vmcnt<0>();  // this wave's residual DMAs have landed (each wave reads only its own slab)
+  // The tile leaves through LDS, each wave's 16 WI x 16 WJ part on its own, so
+  // that the stores are 16 bytes a lane along the rows; rows that are not
+  // 16-byte aligned are stored 8 bytes a lane straight from the accumulators.
+  const bool wide = ((uintptr_t)y & 15) == 0 && (ldy & 7) == 0 && (N & 7) == 0;
+  constexpr int LDW = 32 * WJ + 16;  // bytes per staged row; the pad spreads the rows over the banks
+  static_assert(4 * 16 * WI * LDW <= S * C::STAGE, "the staged tile fits the stages");
+  uint8_t* slab = smem + wave * (16 * WI * LDW);
+  barrier_lds();  // every wave is done reading the stages
+#pragma unroll
+  for (int i = 0; i < WI; ++i) {
+    const int m = m0 + wm * 16 * WI + 16 * i + r16;
+#pragma unroll
+    for (int j = 0; j < WJ; ++j) {
+      const int c = wn * 16 * WJ + 16 * j + 4 * g, n = n0 + c;
+      const u32x2 bb = *reinterpret_cast<const u32x2*>(sbias + c);
       float v[4] = {bf16_to_f32(bb.x & 0xFFFFu), bf16_to_f32(bb.x >> 16), bf16_to_f32(bb.y & 0xFFFFu),
                     bf16_to_f32(bb.y >> 16)};
 #pragma unroll
@@ -315,29 +432,42 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_bf16_kernel(
         v[r] = t;
       }
       if constexpr (RESID) {
-        const u32x2 rr = *reinterpret_cast<const u32x2*>(resid + (int64_t)m * ldr + n);
+        u32x2 rr{0u, 0u};
+        if (rdma) rr = *reinterpret_cast<const u32x2*>(smem + S * C::STAGE + wave * (RQ * 1024) +
+                                                       (16 * i + r16) * (32 * WJ) + (16 * j + 4 * g) * 2);
+        else if (m < M && n < N) rr = *reinterpret_cast<const u32x2*>(resid + (int64_t)m * ldr + n);
         v[0] += bf16_to_f32(rr.x & 0xFFFFu);
         v[1] += bf16_to_f32(rr.x >> 16);
         v[2] += bf16_to_f32(rr.y & 0xFFFFu);
         v[3] += bf16_to_f32(rr.y >> 16);
       }
-      *reinterpret_cast<u32x2*>(y + (int64_t)m * ldy + n) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      const u32x2 o{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      if (wide) *reinterpret_cast<u32x2*>(slab + (16 * i + r16) * LDW + (16 * j + 4 * g) * 2) = o;
+      else if (m < M && n < N) *reinterpret_cast<u32x2*>(y + (int64_t)m * ldy + n) = o;  // N % 4 == 0
     }
+  }
+  if (!wide) return;
+  constexpr int RCH = 2 * WJ;  // 16-byte pieces per row
+#pragma unroll
+  for (int q = 0; q < (16 * WI * RCH + 63) / 64; ++q) {
+    const int e = 64 * q + lane, row = e / RCH, ch = e % RCH;
+    const int m = m0 + wm * 16 * WI + row, n = n0 + wn * 16 * WJ + 8 * ch;
+    if (row < 16 * WI && m < M && n < N)
+      *reinterpret_cast<u32x4*>(y + (int64_t)m * ldy + n) = *reinterpret_cast<const u32x4*>(slab + row * LDW + 16 * ch);
   }
 }
 
-// ---------------------------------------------------------------- packed-weight bf16 GEMM
+// ---------------------------------------------------------------- packed-weight bf16 GEMM, split along k
 //
-// The product and epilogue of gemm_bf16_kernel with the weight read from a
-// setup-time copy in MFMA operand order (ff_pack_weight_bf16) straight into
-// registers, so that only the activations go through LDS. A workgroup of 4
-// waves owns BM rows x BN = 4 CW columns; wave w owns columns [w CW, (w + 1)
-// CW) and all BM rows, so each weight fragment feeds BM / 16 MFMAs and each
-// activation fragment read from LDS CW / 16. A step is 128 k (256 bytes of an
-// activation row, halves h = 0, 1); its four MFMAs per (i, j), sub = 2 h + s,
-// take k 128 kt + 64 h + 16 g + 8 s .. + 8 for lane (r, g): the k partition
-// and order of gemm_bf16_kernel's two MFMAs per 64-k stage, so the
-// accumulators and y are bit-identical to it.
+// For calls too short to fill the GPU: the weight is read from a setup-time copy
+// in MFMA operand order (ff_pack_weight_bf16) straight into registers, so that
+// only the activations go through LDS. A workgroup of 4 waves owns BM rows x BN =
+// 4 CW columns of one k range; wave w owns columns [w CW, (w + 1) CW) and all BM
+// rows, so each weight fragment feeds BM / 16 MFMAs and each activation fragment
+// read from LDS CW / 16. A step is 128 k (256 bytes of an activation row, halves h
+// = 0, 1); its four MFMAs per (i, j), sub = 2 h + s, take k 128 kt + 64 h + 16 g +
+// 8 s .. + 8 for lane (r, g): the k partition and order of gemm_bf16_kernel's two
+// MFMAs per 64-k stage.
 //
 // Activations: two LDS stages of BM rows x 256 bytes, written from registers
 // loaded a step ahead (16-byte chunk c of row r at half c / 8, 1 KB block r / 8,
@@ -346,18 +476,18 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_bf16_kernel(
 // the 16 bytes of row 16 f + r at k 128 kt + 64 (sub / 2) + 16 g + 8 (sub % 2).
 // Each lane holds two steps of fragments in registers; fragment (j, sub) of
 // step kt is reloaded with step kt + 2's right after its MFMAs issue.
+//
+// Workgroup (tile, split) runs k steps [split KT / S, (split + 1) KT / S) and
+// stores its fp32 sums, row-major over the rows padded to whole tiles, at
+// part[(split tiles_m BM + row) N + col]; the launch that follows adds the S
+// partials in split order and applies the epilogue (bf16_split_reduce_kernel, or
+// layer_norm_kernel<true>).
 constexpr int kBfStep = 128;  // k per step of the packed kernel
 
-// PART (k split): workgroup (tile, split) runs k steps [split KT / S, (split
-// + 1) KT / S) and stores its fp32 sums, row-major over the rows padded to
-// whole tiles, at part[(split tiles_m BM + row) N + col] instead of y; the
-// launch that follows adds the S partials in split order and applies the
-// epilogue (bf16_split_reduce_kernel, or layer_norm_kernel<true>).
-template <int BM, int CW, int ACT, bool RESID, bool PART = false>
+template <int BM, int CW>
 __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_pk_kernel(
-    const bf16_t* __restrict__ a, int64_t lda, const uint8_t* __restrict__ wp, const bf16_t* __restrict__ bias,
-    bf16_t* y, int64_t ldy, const bf16_t* resid, int64_t ldr, int M, int N, int K, int tiles_m, int tiles_n,
-    int splits = 1, float* __restrict__ part = nullptr) {
+    const bf16_t* __restrict__ a, int64_t lda, const uint8_t* __restrict__ wp, int M, int N, int K, int tiles_m,
+    int tiles_n, int splits, float* __restrict__ part) {
   constexpr int RA = BM / 16, TJ = CW / 16;
   constexpr int A_CHUNKS = BM * 16;  // 16-byte chunks of one stage
   constexpr int FULL = A_CHUNKS / kThreads, REM = A_CHUNKS % kThreads;
@@ -365,18 +495,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_pk_kernel(
   constexpr int HALF = BM * 128, STAGE = 2 * HALF;
   static_assert(A_CHUNKS >= kThreads, "at least one full activation round");
   __shared__ __align__(1024) uint8_t smem[2 * STAGE];
-  __shared__ __align__(16) float sbias[PART ? 1 : 4 * CW];  // the tile's bias columns, as fp32
-  // The residual tile (RESID): wave w's BM x CW columns at sres + w BM CW,
-  // row-major, copied in by 16-byte LDS DMA after the prologue's loads so that
-  // the epilogue reads it from LDS. Needs 16-byte aligned rows (resid and ldr);
-  // otherwise the epilogue reads it from global memory.
-  constexpr bool RT = RESID && !PART;
-  constexpr int RCH = CW / 8, RQ = BM * RCH / 64;  // chunks per slab row, DMAs per wave
-  static_assert(BM * RCH % 64 == 0, "whole DMA instructions per slab");
-  __shared__ __align__(16) bf16_t sres[RT ? BM * 4 * CW : 1];
 
-  const int S = PART ? splits : 1;
-  const int nblk = tiles_m * tiles_n * S;
+  const int S = splits, nblk = tiles_m * tiles_n * S;
   int logical = blockIdx.x;
   if (nblk % kXcds == 0) logical = (blockIdx.x % kXcds) * (nblk / kXcds) + blockIdx.x / kXcds;
   const int tm = logical % tiles_m, rest = logical / tiles_m;  // M fastest: an XCD's tiles share weight slabs
@@ -434,29 +554,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_pk_kernel(
 #pragma unroll
     for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // The bias is read ahead of the first step (its latency then passes under
-  // the prologue's loads) and kept in LDS for the epilogue.
-  uint32_t braw = 0;
-  if constexpr (!PART)
-    if (tid < 4 * CW) braw = bias[n0 + tid];
   loadA(kt0);
   loadB(kt0, 0);
   writeA(0);
-  if constexpr (!PART)
-    if (tid < 4 * CW) sbias[tid] = bf16_to_f32(braw);
   loadA(min(kt0 + 1, kt1 - 1));
   loadB(min(kt0 + 1, kt1 - 1), 1);
-  const bool rdma = RT && ((uintptr_t)resid & 15) == 0 && (ldr & 7) == 0;
-  if constexpr (RT) {
-    if (rdma) {
-      const uint32_t slab = lds_addr(sres) + (uint32_t)wave_s * (BM * CW * 2);
-#pragma unroll
-      for (int q = 0; q < RQ; ++q) {
-        const int c = 64 * q + lane, row = c / RCH, ch = c % RCH;
-        lds_dma16(resid + (int64_t)min(m0 + row, M - 1) * ldr + n0 + wave * CW + 8 * ch, slab + 1024u * q);
-      }
-    }
-  }
 
   const int frag = 128 * (r16 & 7) + 1024 * (r16 >> 3);
   const int cA[2] = {16 * ((2 * g) ^ (r16 >> 1)), 16 * ((2 * g + 1) ^ (r16 >> 1))};
@@ -504,48 +606,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_pk_kernel(
     });
   }
 
-  // lane (r16, g) of fragment (i, j): row m0 + 16 i + r16, columns
-  // n0 + wave CW + 16 j + 4 g .. + 3; the epilogue of gemm_bf16_kernel
-  if constexpr (PART) {
-    float* dst = part + ((int64_t)split * tiles_m * BM + m0 + r16) * N + n0 + wave * CW + 4 * g;
+  // lane (r16, g) of fragment (i, j): row m0 + 16 i + r16, columns n0 + wave CW + 16 j + 4 g .. + 3
+  float* dst = part + ((int64_t)split * tiles_m * BM + m0 + r16) * N + n0 + wave * CW + 4 * g;
 #pragma unroll
-    for (int i = 0; i < RA; ++i)
+  for (int i = 0; i < RA; ++i)
 #pragma unroll
-      for (int j = 0; j < TJ; ++j) *reinterpret_cast<f32x4*>(dst + (int64_t)16 * i * N + 16 * j) = acc[i][j];
-    return;
-  }
-  if constexpr (RT)
-    if (rdma) {
-      wait_vmcnt<0>();  // this wave's residual DMAs have landed (each wave reads only its own slab)
-      asm volatile("" : : : "memory");
-    }
-#pragma unroll
-  for (int i = 0; i < RA; ++i) {
-    const int m = m0 + 16 * i + r16;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-      const int n = n0 + wave * CW + 16 * j + 4 * g;
-      const f32x4 bv = *reinterpret_cast<const f32x4*>(sbias + n - n0);
-      float v[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float t = round_bf16(acc[i][j][r] + bv[r]);
-        if constexpr (ACT == kGeluTanh) t = round_bf16(gelu_tanh(t));
-        if constexpr (ACT == kGeluErf) t = round_bf16(gelu_erf(t));
-        v[r] = t;
-      }
-      if constexpr (RESID) {
-        const u32x2 rr = rdma ? *reinterpret_cast<const u32x2*>(sres + (wave * BM + 16 * i + r16) * CW + 16 * j + 4 * g)
-                              : *reinterpret_cast<const u32x2*>(resid + (int64_t)m * ldr + n);
-        v[0] += bf16_to_f32(rr.x & 0xFFFFu);
-        v[1] += bf16_to_f32(rr.x >> 16);
-        v[2] += bf16_to_f32(rr.y & 0xFFFFu);
-        v[3] += bf16_to_f32(rr.y >> 16);
-      }
-      *reinterpret_cast<u32x2*>(y + (int64_t)m * ldy + n) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    }
-  }
+    for (int j = 0; j < TJ; ++j) *reinterpret_cast<f32x4*>(dst + (int64_t)16 * i * N + 16 * j) = acc[i][j];
 }
 
 // The epilogue of gemm_bf16_kernel on a k-split launch's S fp32 partial rows
@@ -790,71 +856,88 @@ __global__ __launch_bounds__(kThreads) void pos_interp_kernel(const bf16_t* __re
   *reinterpret_cast<u32x4*>(out + p * hidden + c) = pack8(acc);
 }
 
-template <int BM, int BN, int S, int OCC>
-int launch_gemm(const void* a, int64_t lda, const void* w, const void* bias, void* y, int64_t ldy, const void* resid,
-                int64_t ldr, int64_t m, int64_t n, int64_t k, int act, hipStream_t st) {
-  const int tiles_m = (int)((m + BM - 1) / BM), tiles_n = (int)((n + BN - 1) / BN);
-  const dim3 grid((unsigned)(tiles_m * tiles_n)), block(kThreads);
-#define FF_G(ACT, RES)                                                                                          \
-  if (act == ACT && (resid != nullptr) == RES)                                                                  \
-    hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, S, OCC, ACT, RES>), grid, block, 0, st, (const bf16_t*)a, lda, \
-                       (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, ldy, (const bf16_t*)resid, ldr, (int)m, \
-                       (int)n, (int)k, tiles_m, tiles_n);
-  FF_G(kActNone, false) FF_G(kActNone, true) FF_G(kGeluTanh, false) FF_G(kGeluErf, false)
-#undef FF_G
-  return FF_OK;
-}
+struct GemmArgs {
+  const void *a, *w, *bias, *resid;
+  void* y;
+  int64_t lda, ldy, ldr, m, n, k;
+  int act;
+};
 
-// Tile of the packed kernel for an m x n GEMM: the first (BM, CW) of
-// (128, 48), (64, 64), (64, 48), (64, 32) whose BN = 4 CW divides n and whose
-// grid of 192 .. 256 workgroups runs in one round at one workgroup per CU; 0
-// if none (the LDS-staged kernel then runs). Grids past one round lose to it:
-// the tower's qkv (288 tiles of 128 x 192) took 43.7 us against 28.5, fc1
-// (544 of 64 x 256) 69.2 against 51.0; one-round grids win: proj / fc2 (192
-// of 64 x 192) 30.1 against 32.9 us, the merger's fc1 50.8 against 57.1 and
-// fc2 (256 of 64 x 128) 33.4 against 37.2. (128, 64) would spill: two steps
-// of its weight fragments, two sets of activation fragments and the staging
-// registers exceed the 256 VGPRs.
-int bf16pk_tile(int64_t m, int64_t n) {
-  constexpr int cand[4][2] = {{128, 48}, {64, 64}, {64, 48}, {64, 32}};
-  for (int c = 0; c < 4; ++c) {
-    if (n % (4 * cand[c][1])) continue;
-    const int64_t tiles = (m + cand[c][0] - 1) / cand[c][0] * (n / (4 * cand[c][1]));
-    if (tiles >= 192 && tiles <= 256) return c + 1;
+// One launch of the 32 WI x 32 WJ tile. The stages take what LDS they can use
+// (at most 6), with the residual tile beside them where there is one.
+template <int WI, int WJ>
+void launch_gemm(const GemmArgs& g, hipStream_t st) {
+  constexpr int STAGE = PipeCfg<WI, WJ>::STAGE, LDS = 159 * 1024, RES = 32 * WI * 32 * WJ * 2;
+  constexpr int S0 = LDS / STAGE, S = S0 > 6 ? 6 : S0;
+  constexpr int R0 = (LDS - RES) / STAGE, SR = R0 > 6 ? 6 : R0;
+  const int tiles_m = (int)((g.m + 32 * WI - 1) / (32 * WI)), tiles_n = (int)((g.n + 32 * WJ - 1) / (32 * WJ));
+  const dim3 grid((unsigned)(tiles_m * tiles_n)), block(kThreads);
+  // Strips of tile rows: an XCD reads about m / strips activation rows and n strips / 8 weight rows.
+  int strips = 1;
+  for (int c = 2; c <= 8; c *= 2)
+    if (c <= tiles_m && 8 * g.m / c + g.n * c < 8 * g.m / strips + g.n * strips) strips = c;
+#define FF_G(ACT, RES_, SS)                                                                                        \
+  if (g.act == ACT && (g.resid != nullptr) == RES_)                                                                \
+    hipLaunchKernelGGL((gemm_bf16_kernel<WI, WJ, SS, ACT, RES_>), grid, block, 0, st, (const bf16_t*)g.a, g.lda,   \
+                       (const bf16_t*)g.w, (const bf16_t*)g.bias, (bf16_t*)g.y, g.ldy, (const bf16_t*)g.resid,     \
+                       g.ldr, (int)g.m, (int)g.n, (int)g.k, tiles_m, tiles_n, strips);
+  FF_G(kActNone, false, S) FF_G(kGeluTanh, false, S) FF_G(kGeluErf, false, S)
+  if constexpr (WI * WJ % 2 == 0 && SR >= 3) {
+    FF_G(kActNone, true, SR)
   }
-  return 0;
-}
-
-template <int BM, int CW>
-void launch_gemm_pk(const void* a, int64_t lda, const void* wp, const void* bias, void* y, int64_t ldy,
-                    const void* resid, int64_t ldr, int64_t m, int64_t n, int64_t k, int act, hipStream_t st) {
-  const int tiles_m = (int)((m + BM - 1) / BM), tiles_n = (int)(n / (4 * CW));
-  const dim3 grid((unsigned)(tiles_m * tiles_n)), block(kThreads);
-#define FF_G(ACT, RES)                                                                                         \
-  if (act == ACT && (resid != nullptr) == RES)                                                                 \
-    hipLaunchKernelGGL((gemm_bf16_pk_kernel<BM, CW, ACT, RES>), grid, block, 0, st, (const bf16_t*)a, lda,     \
-                       (const uint8_t*)wp, (const bf16_t*)bias, (bf16_t*)y, ldy, (const bf16_t*)resid, ldr,    \
-                       (int)m, (int)n, (int)k, tiles_m, tiles_n);
-  FF_G(kActNone, false) FF_G(kActNone, true) FF_G(kGeluTanh, false) FF_G(kGeluErf, false)
 #undef FF_G
 }
 
-// k split of the packed GEMM for grids with no one-round tile (bf16pk_tile 0)
-// whose unsplit fallback, 64 x 128 tiles, fills less than half the GPU (the
-// tower at short patch counts, e.g. 400 patches: proj and fc2 have 63 such
-// tiles, the mergers 72; its qkv, 189, runs unsplit: 13.9 us against 15.0 +
-// 4.9 us split 2 ways): the (BM, CW) tile and split count S in {2, 3, 4, 8}
-// whose grid of tiles x S workgroups lies in 192 .. 256 (one round at one per
-// CU) with the least work per workgroup (k steps per split x BM x CW); s = 0
-// when none. ff_set_tuning(FF_TUNE_BF16_PK_SPLIT, 1) turns splits off, 2 .. 8
-// forces the split count.
+// Tile of ff_gemm_bf16: the one with the least rounds x (fixed + stages x step),
+// one workgroup per CU. fixed and step are hundredths of us per launch and per
+// 64-k stage, from 300 x 256 x 192 (one stage time aside) and from pairs of k at
+// one grid (2048 x 1152 and 512 x 4096 rows x columns, k 1152 to 4608), e.g. 96 x
+// 128: 3.7 + 0.445 us per stage, 192 x 192: 6.2 + 0.95. What it decides: the
+// tower at 2048 patches runs fc1 on 192 x 192 (28.5 us; 96 x 192 35.1), qkv on
+// 160 x 192 (21.6; 192 x 192 23.0), proj on 96 x 128 or 64 x 160 (13.2 - 13.7), fc2
+// on 96 x 128 (36.0; 64 x 160 38.2); at 400 patches qkv on 64 x 96 (10.0; 64 x 128
+// 11.4), fc1 on 64 x 128 (12.3; 96 x 128 13.7). The residual add needs room for
+// its tile beside three stages, which the last two do not leave.
+// ff_set_tuning(FF_TUNE_GEMM_BF16_TILE, 10 WI + WJ) forces a tile of the list.
+struct TileCost {
+  int wi, wj, fixed, step;
+};
+constexpr TileCost kTiles[] = {{1, 2, 250, 17}, {2, 2, 270, 29}, {2, 3, 295, 34}, {2, 4, 310, 42}, {2, 5, 340, 49},
+                               {3, 4, 365, 45}, {4, 4, 400, 57}, {3, 6, 440, 60}, {5, 6, 570, 81}, {6, 6, 620, 95}};
+constexpr int kResidTiles = 8;  // the first of them that take a residual
+
+int bf16_tile(int64_t m, int64_t n, int64_t k, bool resid) {
+  const int nt = resid ? kResidTiles : (int)(sizeof(kTiles) / sizeof(kTiles[0]));
+  const int forced = ff_tuning(FF_TUNE_GEMM_BF16_TILE);
+  int best = 0;
+  int64_t best_cost = 0;
+  for (int i = 0; i < nt; ++i) {
+    const TileCost& t = kTiles[i];
+    if (forced == 10 * t.wi + t.wj) return i;
+    const int64_t tiles = (m + 32 * t.wi - 1) / (32 * t.wi) * ((n + 32 * t.wj - 1) / (32 * t.wj));
+    const int64_t cost = (tiles + 255) / 256 * (t.fixed + k / 64 * t.step);
+    if (i == 0 || cost < best_cost) {
+      best = i;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+// k split of the packed GEMM for calls whose 64 x 128 tiles fill less than half
+// the GPU (the tower at short patch counts, e.g. 400 patches: proj and fc2 have 63
+// such tiles, the mergers 72): the (BM, CW) tile and split count S in {2, 3, 4, 8}
+// whose grid of tiles x S workgroups lies in 192 .. 256 (one round at one per CU)
+// with the least work per workgroup (k steps per split x BM x CW); s = 0 when
+// none. ff_set_tuning(FF_TUNE_BF16_PK_SPLIT, 1) turns splits off, 2 .. 8 forces
+// the split count.
 struct Bf16Split {
   int bm = 0, cw = 0, s = 0;
 };
 Bf16Split bf16pk_split(int64_t m, int64_t n, int64_t k) {
   Bf16Split p;
   const int forced = ff_tuning(FF_TUNE_BF16_PK_SPLIT);
-  if (forced == 1 || m <= 0 || k % kBfStep || bf16pk_tile(m, n)) return p;
+  if (forced == 1 || m <= 0 || k % kBfStep) return p;
   if (!forced && (m + 63) / 64 * ((n + 127) / 128) >= 128) return p;
   const int64_t kt = k / kBfStep;
   constexpr int cand[4][2] = {{64, 32}, {64, 48}, {64, 64}, {128, 48}};
@@ -883,9 +966,9 @@ template <int BM, int CW>
 void launch_gemm_pk_part(const void* a, int64_t lda, const void* wp, int64_t m, int64_t n, int64_t k, int splits,
                          void* part, hipStream_t st) {
   const int tiles_m = (int)((m + BM - 1) / BM), tiles_n = (int)(n / (4 * CW));
-  hipLaunchKernelGGL((gemm_bf16_pk_kernel<BM, CW, kActNone, false, true>), dim3((unsigned)(tiles_m * tiles_n * splits)),
-                     dim3(kThreads), 0, st, (const bf16_t*)a, lda, (const uint8_t*)wp, nullptr, nullptr, 0, nullptr, 0,
-                     (int)m, (int)n, (int)k, tiles_m, tiles_n, splits, (float*)part);
+  hipLaunchKernelGGL((gemm_bf16_pk_kernel<BM, CW>), dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(kThreads), 0, st,
+                     (const bf16_t*)a, lda, (const uint8_t*)wp, (int)m, (int)n, (int)k, tiles_m, tiles_n, splits,
+                     (float*)part);
 }
 
 // The split GEMM's partials for plan p (the packed kernel's conditions and the
@@ -951,22 +1034,19 @@ extern "C" int ff_gemm_bf16(const void* a, int64_t lda, const void* w, const voi
                  (!resid || ff_aligned(resid, 8)),
              "ff_gemm_bf16: alignment");
   hipStream_t st = (hipStream_t)stream;
-  const int64_t big = ((m + 127) / 128) * ((n + 127) / 128);
-  // ff_set_tuning(FF_TUNE_GEMM_BF16_TILE, 1..3) forces 64x128 | 128x128 | 64x128 at three per CU.
-  const int forced = ff_tuning(FF_TUNE_GEMM_BF16_TILE) - 1;
-  // 128 x 128 tiles at two workgroups per CU when they fill at least three
-  // quarters of the 512 slots, else 64 x 128 tiles (more workgroups for the
-  // narrow projections). The GELU-tanh MLP input projection (the tower's fc1,
-  // 2048 x 1152 -> 4352 at 2048 patches) runs 64 x 128 tiles at three per CU
-  // instead: 42.7 us against 51.5 (128 x 128) and 50.3 (64 x 128, two per CU),
-  // its VALU-heavy epilogue overlapping the other workgroups' main loops.
-  const int tile = forced >= 0 ? forced : (big >= 384 ? (act == kGeluTanh ? 2 : 1) : 0);
-  if (tile == 1)
-    launch_gemm<128, 128, 2, 2>(a, lda, w, bias, y, ldy, resid, ldr, m, n, k, act, st);
-  else if (tile == 2)
-    launch_gemm<64, 128, 2, 3>(a, lda, w, bias, y, ldy, resid, ldr, m, n, k, act, st);
-  else
-    launch_gemm<64, 128, 3, 2>(a, lda, w, bias, y, ldy, resid, ldr, m, n, k, act, st);
+  const GemmArgs g{a, w, bias, resid, y, lda, ldy, ldr, m, n, k, act};
+  switch (bf16_tile(m, n, k, resid != nullptr)) {
+    case 0: launch_gemm<1, 2>(g, st); break;
+    case 1: launch_gemm<2, 2>(g, st); break;
+    case 2: launch_gemm<2, 3>(g, st); break;
+    case 3: launch_gemm<2, 4>(g, st); break;
+    case 4: launch_gemm<2, 5>(g, st); break;
+    case 5: launch_gemm<3, 4>(g, st); break;
+    case 6: launch_gemm<4, 4>(g, st); break;
+    case 7: launch_gemm<3, 6>(g, st); break;
+    case 8: launch_gemm<5, 6>(g, st); break;
+    default: launch_gemm<6, 6>(g, st); break;
+  }
   FF_LAUNCH_CHECK("ff_gemm_bf16");
   return FF_OK;
 }
@@ -986,28 +1066,8 @@ extern "C" int ff_pack_weight_bf16(const void* w, void* packed, int64_t n, int64
 extern "C" int ff_gemm_bf16_pk(const void* a, int64_t lda, const void* w, const void* w_packed, const void* bias,
                                void* y, int64_t ldy, const void* resid, int64_t ldr, int64_t m, int64_t n, int64_t k,
                                int act, ff_stream_t stream) {
-  const int tile = w_packed && k % kBfStep == 0 && ff_aligned(w_packed, 16) && ff_aligned(a, 16) &&
-                           m * lda * 2 < (int64_t(1) << 31) && n * k * 2 < (int64_t(1) << 31)
-                       ? bf16pk_tile(m, n)
-                       : 0;
-  if (tile == 0) return ff_gemm_bf16(a, lda, w, bias, y, ldy, resid, ldr, m, n, k, act, stream);
-  FF_REQUIRE(a && w && bias && y, "ff_gemm_bf16_pk: null pointer");
-  FF_REQUIRE(m > 0 && lda >= k && ldy >= n && lda % 8 == 0 && ldy % 4 == 0 && (!resid || (ldr >= n && ldr % 4 == 0)),
-             "ff_gemm_bf16_pk: bad sizes m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
-  FF_REQUIRE(act == kActNone || act == kGeluTanh || act == kGeluErf, "ff_gemm_bf16_pk: act %d unknown", act);
-  FF_REQUIRE(!resid || act == kActNone, "ff_gemm_bf16_pk: a residual add takes no activation");
-  FF_REQUIRE(ff_aligned(bias, 8) && ff_aligned(y, 8) && (!resid || ff_aligned(resid, 8)), "ff_gemm_bf16_pk: alignment");
-  hipStream_t st = (hipStream_t)stream;
-  if (tile == 1)
-    launch_gemm_pk<128, 48>(a, lda, w_packed, bias, y, ldy, resid, ldr, m, n, k, act, st);
-  else if (tile == 2)
-    launch_gemm_pk<64, 64>(a, lda, w_packed, bias, y, ldy, resid, ldr, m, n, k, act, st);
-  else if (tile == 3)
-    launch_gemm_pk<64, 48>(a, lda, w_packed, bias, y, ldy, resid, ldr, m, n, k, act, st);
-  else
-    launch_gemm_pk<64, 32>(a, lda, w_packed, bias, y, ldy, resid, ldr, m, n, k, act, st);
-  FF_LAUNCH_CHECK("ff_gemm_bf16_pk");
-  return FF_OK;
+  (void)w_packed;  // only the k split of the workspace entry points reads it
+  return ff_gemm_bf16(a, lda, w, bias, y, ldy, resid, ldr, m, n, k, act, stream);
 }
 
 extern "C" int ff_gemm_bf16_pk_workspace(int64_t m, int64_t n, int64_t k, int64_t* bytes) {

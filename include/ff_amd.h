@@ -39,7 +39,8 @@ int ff_device_check(void);
  * ff_set_tuning runs the built-in choices. Set them only while no launch of an
  * affected entry point is being issued from another thread. */
 #define FF_TUNE_GEMM_FP8_TILE 1   /* ff_gemm_fp8 / _qkv: 1 64x128, 2 128x128, 3 128x128 4-stage, 4 128x256 */
-#define FF_TUNE_GEMM_BF16_TILE 2  /* ff_gemm_bf16: 1 64x128, 2 128x128, 3 64x128 at three per CU */
+#define FF_TUNE_GEMM_BF16_TILE 2  /* ff_gemm_bf16: 10 WI + WJ (32 WI x 32 WJ tile): 12, 22, 23, 24, 25, 34, 44, 36,
+                                     56 or 66 (the last two not with a residual) */
 #define FF_TUNE_W4A16_TILE 3      /* ff_gemm_w4a16*: 1 64x256, 2 192x192 */
 #define FF_TUNE_W4A16_SPLITS 4    /* ff_gemm_w4a16_ws: k splits of the 64x256 tile, 1..8 */
 #define FF_TUNE_ATTN_QT 5         /* ff_attention_vt prefill (1, 2 or 4) / ff_attention_full (1 or 2): query tiles per wave */
@@ -486,12 +487,10 @@ int ff_gemm_bf16(const void* a, int64_t lda, const void* w, const void* bias, vo
  * 64 (s / 2) + 16 g + 8 (s % 2). packed holds 2 n k bytes. n % 16 == 0,
  * k % 128 == 0. */
 int ff_pack_weight_bf16(const void* w, void* packed, int64_t n, int64_t k, ff_stream_t stream);
-/* ff_gemm_bf16 with the weight read from its packed copy (ff_pack_weight_bf16
- * of w) straight into the matrix-core operands: the same products in the same
- * order, so the same bits. Taken when w_packed is given, k % 128 == 0 and a
- * tile of 128 x 192, 64 x 256, 64 x 192 or 64 x 128 divides n and gives a grid
- * of 192..256 workgroups; otherwise this is ff_gemm_bf16 on w (w_packed may be
- * NULL). Same reference replacement as ff_gemm_bf16. */
+/* ff_gemm_bf16 of a caller that also holds the weight's packed copy
+ * (ff_pack_weight_bf16 of w; may be NULL): the unsplit product, the same bits.
+ * The copy is read by the k split of the workspace entry points below. Same
+ * reference replacement as ff_gemm_bf16. */
 int ff_gemm_bf16_pk(const void* a, int64_t lda, const void* w, const void* w_packed, const void* bias, void* y,
                     int64_t ldy, const void* resid, int64_t ldr, int64_t m, int64_t n, int64_t k, int act,
                     ff_stream_t stream);
@@ -499,9 +498,9 @@ int ff_gemm_bf16_pk(const void* a, int64_t lda, const void* w, const void* w_pac
 /* Bytes of workspace ff_gemm_bf16_pk_ws / ff_gemm_bf16_pk_ln need for an
  * m x n x k product (0: it runs unsplit). Host-only. */
 int ff_gemm_bf16_pk_workspace(int64_t m, int64_t n, int64_t k, int64_t* bytes);
-/* ff_gemm_bf16_pk with a k split where the packed kernel has no tile whose
- * grid fills the GPU in one round (short m: the tower at 400 patches, the
- * patch mergers): the split launches store fp32 partials in workspace
+/* ff_gemm_bf16_pk with a k split, on the packed copy, where 64 x 128 tiles would
+ * fill less than half the GPU (short m: the tower at 400 patches, the patch
+ * mergers): the split launches store fp32 partials in workspace
  * (ff_gemm_bf16_pk_workspace bytes, 16-byte aligned) and a second launch adds
  * them in split order and applies the epilogue (bias, act, resid). The same
  * products summed in another order: within an fp32 rounding of the unsplit

@@ -126,6 +126,66 @@ def test_gemm_bf16_residual_in_place(gpu):
     _assert_within(hd.cpu(), want, bound, "gemm_bf16 residual")
 
 
+FF_TUNE_GEMM_BF16_TILE = 2
+BF16_TILES = [12, 22, 23, 24, 25, 34, 44, 36, 56, 66]
+
+
+# one row and one column group; ragged rows and columns around the tiles' edges
+# (32, 64, 96, 160, 192), a row of outputs that is not 16-byte aligned (n % 8 ==
+# 4); one 64-k stage, fewer stages than are in flight, as many, and many more
+@pytest.mark.parametrize("m,n,k", [(1, 4, 64), (33, 100, 128), (191, 196, 384), (193, 320, 448), (385, 1160, 1152)])
+def test_gemm_bf16_every_tile(gpu, m, n, k):
+    """ff_gemm_bf16 with each tile forced: bit-equal to the first one (the same
+    products in the same order), which is inside the fp32-accumulation bound; the
+    same for each activation and for a residual added in place."""
+    from fastforward_amd._lib import call
+    from fastforward_amd.vision import Lin, linear
+    x = torch.randn(m, k, generator=_g(m + 21)).to(BF16)
+    w = (torch.randn(n, k, generator=_g(n + 22)) * 0.05).to(BF16)
+    b = (torch.randn(n, generator=_g(k + 23)) * 0.1).to(BF16)
+    h = torch.randn(m, n, generator=_g(24)).to(BF16).to(DEV)
+    xd, lin = x.to(DEV), Lin(w.to(DEV), b.to(DEV))
+
+    def run(tile):
+        call("ff_set_tuning", FF_TUNE_GEMM_BF16_TILE, tile)
+        try:
+            y = h.clone()
+            linear(xd, lin, resid=y, out=y)
+            return [linear(xd, lin, act=act) for act in (0, 1, 2)] + [y]
+        finally:
+            call("ff_set_tuning", FF_TUNE_GEMM_BF16_TILE, 0)
+    ref = run(BF16_TILES[0])
+    exact, bound = _linear_bound(x, w, b)
+    assert bool(((ref[0].cpu().to(torch.float64) - exact).abs() <= bound).all())
+    for tile in BF16_TILES[1:] + [0]:
+        for a, c in zip(run(tile), ref):
+            assert torch.equal(a, c), tile
+
+
+def test_gelu_tanh_every_bf16(gpu):
+    """The GELU-tanh epilogue at every finite bf16 value (an identity weight
+    carries x to the epilogue exactly): within one bf16 ulp of the 64-bit function,
+    plus 2^-24 |x| where the result itself is below that (the fp32 evaluation's
+    absolute floor), and infinities and NaN as torch's."""
+    from fastforward_amd.vision import Lin, linear
+    bits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF16)
+    vals = bits[torch.isfinite(bits.float())]
+    vals = torch.cat([vals, torch.zeros((-vals.numel()) % 64)]).to(BF16).reshape(-1, 64)
+    eye = torch.eye(64).to(BF16)
+    got = linear(vals.to(DEV), Lin(eye.to(DEV), torch.zeros(64, dtype=BF16, device=DEV)), act=1).cpu()
+    v = vals.to(torch.float64)
+    u = (2 / np.pi) ** 0.5 * (v + 0.044715 * v ** 3)
+    want = v / (1 + torch.exp(-2 * u))
+    ok = (got.to(torch.float64) - want).abs() <= _ulp(want) + v.abs() * 2.0 ** -24
+    assert bool(ok.all()), vals[~ok][:8]
+    sp = torch.zeros(1, 64, dtype=BF16)
+    for x, f in ((float("inf"), lambda t: t == float("inf")), (float("nan"), torch.isnan)):
+        sp[0, 0] = x
+        out = linear(sp.to(DEV), Lin(eye.to(DEV)[:, :64].contiguous(), torch.zeros(64, dtype=BF16, device=DEV)),
+                     act=1).cpu()
+        assert bool(f(out[0, 0].float()))
+
+
 # (m, k, n, act, resid): proj / fc2 of the tower with the residual add in place
 # (64 x 192 tiles), the patch embedding, the mergers' fc1 + GELU (64 x 192) and
 # fc2 (64 x 128), the 128 x 192 and 64 x 256 tiles (GELU-tanh) at row counts
