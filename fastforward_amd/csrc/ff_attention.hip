@@ -94,6 +94,22 @@ __global__ __launch_bounds__(kThreads) void qkv_post_kernel(
 // Both kernels share the per-block softmax below, so they produce identical
 // bits for the same query.
 
+// Maximum of matrix-unit results: NaN propagates (a NaN score makes the whole
+// row NaN either way), so the compiler needs no canonicalising v_max per score,
+// which fmaxf takes (16 of the 26 instructions of a block's maximum).
+__device__ __forceinline__ float fmax_nc(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
+// Maximum of a lane's 16 scores.
+__device__ __forceinline__ float max16(const f32x4 (&s)[4]) {
+  float r = fmax_nc(fmax_nc(s[0][0], s[0][1]), s[0][2]);
+  r = fmax_nc(fmax_nc(r, s[0][3]), s[1][0]);
+  float u = fmax_nc(fmax_nc(s[1][1], s[1][2]), s[1][3]);
+  u = fmax_nc(fmax_nc(u, s[2][0]), s[2][1]);
+  float v = fmax_nc(fmax_nc(s[2][2], s[2][3]), s[3][0]);
+  v = fmax_nc(fmax_nc(v, s[3][1]), s[3][2]);
+  return fmax_nc(fmax_nc(fmax_nc(r, u), v), s[3][3]);
+}
+
 // One 64-key block of the online softmax for a 16-query tile held as S^T
 // accumulators: s[2c + tt][r] = q.k of key kb + 32c + 8g + 4tt + r for the
 // lane's query (lane (r16, g) = (query, key group)). Keys whose offset
@@ -112,10 +128,7 @@ __device__ __forceinline__ float softmax_block(f32x4 (&s)[4], bool masked, int l
       for (int r = 0; r < 4; ++r)
         if (32 * (i >> 1) + 4 * (i & 1) + r > lim) s[i][r] = -INFINITY;
   }
-  float bmax = fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3]));
-#pragma unroll
-  for (int i = 1; i < 4; ++i) bmax = fmaxf(bmax, fmaxf(fmaxf(s[i][0], s[i][1]), fmaxf(s[i][2], s[i][3])));
-  const float mnew = fmaxf(m, max_rows(bmax));
+  const float mnew = fmaxf(m, max_rows(max16(s)));
   const float mref = mnew == -INFINITY ? 0.f : mnew;  // a fully masked query keeps p = 0, alpha = 0
   const float alpha = __builtin_amdgcn_exp2f((m - mref) * c2);
   float p[16], psum = 0.f;
@@ -139,6 +152,48 @@ __device__ __forceinline__ float softmax_block(f32x4 (&s)[4], bool masked, int l
   return alpha;
 }
 
+// The block of the bidirectional attention (the vision tower), which has no
+// schedule to reproduce: the scores' reference m moves only when some query's
+// maximum exceeds its own by more than 2^8 in p (p then stays below 256, and
+// bf16(p), its sum and the products keep their relative precision), so that
+// after the first block alpha is 1 and acc needs no rescale; and (s - m) c2 is
+// one fma. VALU instructions per 16 scores: 64 instead of 114.
+__device__ __forceinline__ float softmax_block_free(f32x4 (&s)[4], bool masked, int lim, float c2, float& m,
+                                                    float& den, u32x4 (&pf)[2]) {
+  if (masked) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (32 * (i >> 1) + 4 * (i & 1) + r > lim) s[i][r] = -INFINITY;
+  }
+  const float mnew = fmaxf(m, max_rows(max16(s)));
+  float alpha = 1.0f;
+  if (__ballot((mnew - m) * c2 > 8.0f)) {  // m = -inf before the first block
+    alpha = __builtin_amdgcn_exp2f((m - mnew) * c2);
+    m = mnew;
+  }
+  const float off = m == -INFINITY ? 0.f : -m * c2;  // every score so far -inf: p = 0
+  float p[16], psum = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], c2, off));
+      p[4 * i + r] = e;
+      psum += e;
+    }
+  den = den * alpha + psum;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    pf[c].x = pack_bf16x2(p[8 * c + 0], p[8 * c + 1]);
+    pf[c].y = pack_bf16x2(p[8 * c + 2], p[8 * c + 3]);
+    pf[c].z = pack_bf16x2(p[8 * c + 4], p[8 * c + 5]);
+    pf[c].w = pack_bf16x2(p[8 * c + 6], p[8 * c + 7]);
+  }
+  return alpha;
+}
+
 // acc *= alpha (its first DTN 16-column tiles), skipped when no query of the
 // wave changed its max (alpha == 1 exactly leaves acc unchanged).
 template <int DTN = 8>
@@ -149,17 +204,28 @@ __device__ __forceinline__ void rescale(f32x4 (&o)[8], float alpha) {
   }
 }
 
+// x / d correctly rounded from r = 1 / d correctly rounded, with the special cases
+// of the IEEE division (v_div_fixup_f32): a row divides all its values by one
+// denominator, so the reciprocal is taken once (4 instructions per value
+// instead of 12).
+__device__ __forceinline__ float div_den(float x, float d, float r) {
+  const float y = x * r;
+  const float e = __builtin_fmaf(-y, d, x);
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(e, r, y), d, x);
+}
+
 // Output row of one (query, head): o / den as bf16, the first DOUT of the 128
 // head dims (DOUT % 4 == 0; the columns past it are the zero padding of a
 // narrower head).
 template <int DOUT = D>
 __device__ __forceinline__ void store_rows(bf16_t* __restrict__ yp, const f32x4 (&o)[8], float den, int g) {
+  const float r = 1.0f / den;
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt) {
     if (16 * dt + 4 * g >= DOUT) continue;
     u32x2 w2;
-    w2.x = pack_bf16x2(o[dt][0] / den, o[dt][1] / den);
-    w2.y = pack_bf16x2(o[dt][2] / den, o[dt][3] / den);
+    w2.x = pack_bf16x2(div_den(o[dt][0], den, r), div_den(o[dt][1], den, r));
+    w2.y = pack_bf16x2(div_den(o[dt][2], den, r), div_den(o[dt][3], den, r));
     *reinterpret_cast<u32x2*>(yp + 16 * dt + 4 * g) = w2;
   }
 }
@@ -169,11 +235,12 @@ __device__ __forceinline__ void store_rows(bf16_t* __restrict__ yp, const f32x4 
 // output the reference writes, then its runtime-scale cast, 4 bytes per dt.
 __device__ __forceinline__ void store_rows_q(uint8_t* __restrict__ yp, const f32x4 (&o)[8], float den, int g,
                                              float inv) {
+  const float r = 1.0f / den;
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt) {
     *reinterpret_cast<uint32_t*>(yp + 16 * dt + 4 * g) =
-        quant4_static(round_bf16(o[dt][0] / den), round_bf16(o[dt][1] / den), round_bf16(o[dt][2] / den),
-                      round_bf16(o[dt][3] / den), inv);
+        quant4_static(round_bf16(div_den(o[dt][0], den, r)), round_bf16(div_den(o[dt][1], den, r)),
+                      round_bf16(div_den(o[dt][2], den, r)), round_bf16(div_den(o[dt][3], den, r)), inv);
   }
 }
 
@@ -341,10 +408,7 @@ __device__ __forceinline__ float decode_scores(const u32x4 (&kf)[16], const u32x
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (32 * (i >> 1) + 4 * (i & 1) + r > lim) sc[i][r] = -INFINITY;
-  float bmax = fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3]));
-#pragma unroll
-  for (int i = 1; i < 4; ++i) bmax = fmaxf(bmax, fmaxf(fmaxf(sc[i][0], sc[i][1]), fmaxf(sc[i][2], sc[i][3])));
-  return max_rows(bmax);
+  return max_rows(max16(sc));
 }
 
 // Pass 2 for one block: P against the sequential running max mnew of the
@@ -512,13 +576,18 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attention_decode_kernel(
 // CU, 96 KB LDS; NS = 2: two per CU, 64 KB each), and every fragment read
 // from LDS feeds QT MFMAs.
 //
-// LDS stage layout (32 KB): K at [0, 16 KB), V^T at [16 KB, 32 KB), each as
-// sixteen 1 KB blocks of 8 rows x 128 B. K row `key` (0..63 within the block)
-// half h sits in block 2*(key/8) + h, row key%8; V^T row d in block d/8, row
-// d%8. Inside a 128 B row the 16 B chunk c is stored at slot c ^ swz with
-// swz = ((key>>1)&1) | ((key>>2)&6) for K and (d>>1)&7 for V^T, which makes
-// every MFMA fragment read (16 lanes per LDS cycle) hit 16 distinct bank
-// groups.
+// LDS stage layout (32 KB at 128 dims), 1 KB blocks of 8 rows x 128 B: K dims 0 ..
+// 63 of the 64 keys in blocks 0 .. 7 (row `key` in block key/8), dims 64 .. 127 in
+// the next 8, then V^T (row d in block d/8). Inside a 128 B row the 16 B chunk c is
+// stored at slot c ^ swz with swz = ((key>>1)&1) | ((key>>2)&6) for K and (d>>1)&7
+// for V^T, which makes every MFMA fragment read (16 lanes per LDS cycle) hit 16
+// distinct bank groups. Narrower heads (zero-padded in memory) load only what is
+// computed: at 72 dims K dims 64 .. 95 as 4 blocks of 16 rows x 64 B and 80 rows
+// of V^T, 22 KB.
+//
+// KS = 2 (bidirectional only): two sets of NW waves share the queries, set s takes
+// the key blocks s, s + 2, ..; a stage holds one block of each, and the sets'
+// sums are merged through LDS at the end.
 //
 // Grid: one dimension, heaviest query blocks first across all groups; the
 // group is blockIdx % (hq/HPW), so with 8 XCDs taking workgroups round-robin
@@ -529,15 +598,24 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attention_decode_kernel(
 // head dim stored per (query, head) of y, which is (s, hq, DOUT); heads
 // narrower than 128 are zero-padded to 128 in q, k and V^T, which leaves every
 // score and every stored output column exact.
-template <int QT, int HPW, int NS, bool CAUSAL = true, int DOUT = D, bool QOUT = false>
-__global__ __launch_bounds__(kThreads, NS == 2 ? 2 : 1) void attention_prefill_kernel(
+template <int QT, int HPW, int NS, bool CAUSAL = true, int DOUT = D, bool QOUT = false, int NW = 4, int KS = 1>
+__global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)) void attention_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ vt,
     bf16_t* __restrict__ y, int s_len, int t, int t_pad, int hq, int hk, float c2, int nqb, float qinv) {
-  constexpr int QB = 16 * QT * (4 / HPW);
-  constexpr int STAGE = 32 * 1024;
+  constexpr int QB = 16 * QT * (NW / HPW);
+  // Head dims past DOUT are zero in q, k and V^T: only the first KST 32-dim
+  // steps of q.k and the first DTN 16-dim tiles of P.V are loaded and computed.
+  constexpr int KST = (DOUT + 31) / 32, DTN = (DOUT + 15) / 16;
+  constexpr int KH = KST == 4 ? 8 : (KST == 3 ? 4 : 0);  // 1 KB blocks of K dims 64 and up
+  constexpr int VB = 2 * DTN, BLOCKS = 8 + KH + VB;      // and of V^T, and of a stage
+  constexpr int NT = NW * KS;                            // waves
+  constexpr int PW = (KS * BLOCKS + NT - 1) / NT;        // DMAs per wave and stage
+  constexpr int KB = BLOCKS * 1024, STAGE = KS * KB, VOFF = (8 + KH) * 1024;
   static_assert(NS == 2 || NS == 3, "two or three K/V stages");
+  static_assert(KS == 1 || (!CAUSAL && HPW == 1 && !QOUT), "only the bidirectional attention splits keys over waves");
   __shared__ __align__(1024) uint8_t smem[NS * STAGE];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wid % NW, ks = wid / NW;  // query set, share of the key blocks
   const int r16 = lane & 15, g = lane >> 4;
   const int ngroups = hq / HPW;
   const int grp = (int)blockIdx.x % ngroups;
@@ -547,45 +625,64 @@ __global__ __launch_bounds__(kThreads, NS == 2 ? 2 : 1) void attention_prefill_k
   const int q0 = qb * QB;
   const int wq0 = q0 + (wave / HPW) * 16 * QT;  // first query of this wave
   const int kend = CAUSAL ? min(t, min(s_len, q0 + QB)) : t;  // keys [0, kend) are visible to some query
-  const int nblocks = (kend + 63) / 64;
+  const int nblocks = (kend + 63) / 64, niter = (nblocks + KS - 1) / KS;
 
-  // Load sources of this lane: blocks wave + 4i, i = 0..7 (0..15 K, 16..31 V^T).
+  // Load sources of this lane: the stage's 1 KB blocks id = wid + NT i (past the
+  // last one: the last again, the same bytes to the same place, so that every
+  // wave counts PW loads per stage), id / BLOCKS = which of the stage's KS key
+  // blocks, b = id % BLOCKS: b < 8: K rows [8 b, 8 b + 8), dims 0 .. 63; then dims 64
+  // and up, 8 rows x 128 B (KST 4) or 16 rows x 64 B (KST 3: dims 64 .. 95); then V^T
+  // rows 8 per block. Key blocks past the last one load the last one again.
   const bf16_t* kbase = k + (int64_t)kvh * t * D;
   const bf16_t* vbase = vt + (int64_t)kvh * D * t_pad;
-  int k_key[4], k_col[4];
-  int64_t v_off[4];
+  auto block_of = [&](int i) { return (KS * BLOCKS) % NT ? min(wid + NT * i, KS * BLOCKS - 1) : wid + NT * i; };
+  int k_key[PW], k_col[PW];
+  int64_t v_off[PW];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int bi = wave + 4 * i;  // K block
-    const int key = 8 * (bi >> 1) + (lane >> 3);
+  for (int i = 0; i < PW; ++i) {
+    const int b = block_of(i) % BLOCKS;
+    int key = 8 * (b & 7) + (lane >> 3);
     const int swz = ((key >> 1) & 1) | ((key >> 2) & 6);
+    int col = 64 * (b >> 3) + 8 * ((lane & 7) ^ swz);
+    if (KST == 3 && b >= 8) {
+      key = 16 * (b & 3) + (lane >> 2);
+      col = 64 + 8 * ((lane & 3) ^ ((key >> 3) & 3));
+    }
     k_key[i] = key;
-    k_col[i] = 64 * (bi & 1) + 8 * ((lane & 7) ^ swz);
-    const int d = 8 * bi + (lane >> 3);  // V^T block bi
+    k_col[i] = col;
+    const int d = 8 * (b - 8 - KH) + (lane >> 3);
     v_off[i] = (int64_t)d * t_pad + 8 * ((lane & 7) ^ ((d >> 1) & 7));
   }
-  const uint32_t lds0 = lds_addr(smem) + (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 1024;
-  auto issue = [&](int kb, int buf) {
-    const uint32_t st = lds0 + buf * STAGE;
+  const uint32_t lds0 = lds_addr(smem);
+  auto issue = [&](int it, int buf) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int key = min(kb + k_key[i], t - 1);
-      lds_dma16(kbase + (int64_t)key * D + k_col[i], st + 4 * i * 1024);
+    for (int i = 0; i < PW; ++i) {
+      const int id = block_of(i);  // wave-uniform
+      const int kb = 64 * (KS == 1 ? it : min(KS * it + id / BLOCKS, nblocks - 1));
+      const uint32_t dst = lds0 + buf * STAGE + (uint32_t)id * 1024;
+      // K or V^T, known at compile time where round i holds one kind only
+      const bool isk = KS == 1 && NT * (i + 1) <= 8 + KH ? true
+                       : KS == 1 && NT * i >= 8 + KH     ? false
+                                                         : id % BLOCKS < 8 + KH;
+      if (isk) lds_dma16(kbase + (int64_t)min(kb + k_key[i], t - 1) * D + k_col[i], dst);
+      else lds_dma16(vbase + v_off[i] + kb, dst);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) lds_dma16(vbase + v_off[i] + kb, st + 16 * 1024 + 4 * i * 1024);
   };
 
   // Fragment read offsets (bytes within a stage). K fragment (c, tt, st):
-  // key = 32c + 8(r16>>2) + 4tt + (r16&3), d chunk 4st + g, swz = r16>>1.
+  // key = 32c + 8(r16>>2) + 4tt + (r16&3), d chunk 4st + g, swz = r16>>1 (dims 64
+  // .. 95 of KST 3: chunk g at slot g ^ (key/8 % 4)).
   // V^T fragment (dt, c): d = 16dt + r16, key chunk 4c + g, swz = (r16>>1)&7.
   const int sw = r16 >> 1;
   auto koff = [&](int c, int tt, int st) {
-    return ((4 * c + (r16 >> 2)) * 2 + (st >> 1)) * 1024 + (4 * tt + (r16 & 3)) * 128 +
+    if (KST == 3 && st == 2)
+      return (8 + 2 * c + (r16 >> 3)) * 1024 + (8 * ((r16 >> 2) & 1) + 4 * tt + (r16 & 3)) * 64 +
+             16 * (g ^ (r16 >> 2));
+    return (8 * (st >> 1) + 4 * c + (r16 >> 2)) * 1024 + (4 * tt + (r16 & 3)) * 128 +
            16 * ((4 * (st & 1) + g) ^ sw);
   };
   auto voff = [&](int dt, int c) {
-    return 16 * 1024 + (2 * dt + (r16 >> 3)) * 1024 + (r16 & 7) * 128 + 16 * ((4 * c + g) ^ sw);
+    return VOFF + (2 * dt + (r16 >> 3)) * 1024 + (r16 & 7) * 128 + 16 * ((4 * c + g) ^ sw);
   };
 
   f32x4 o[QT][8];
@@ -601,11 +698,9 @@ __global__ __launch_bounds__(kThreads, NS == 2 ? 2 : 1) void attention_prefill_k
   // The first NS-1 key blocks and the queries load together. The queries are
   // waited for before the loop: a compiler-placed wait for them inside the
   // loop would also wait for the prefetches issued there.
-  issue(0, 0);
-  if (NS == 3 && nblocks > 1) issue(64, 1);
-  // Head dims past DOUT are zero in q, k and V^T: only the first KST 32-dim
-  // steps of q.k and the first DTN 16-dim tiles of P.V are computed.
-  constexpr int KST = (DOUT + 31) / 32, DTN = (DOUT + 15) / 16;
+#pragma unroll
+  for (int st = 0; st < NS - 1; ++st)
+    if (st < niter) issue(st, st);
   u32x4 qf[QT][4];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -620,14 +715,15 @@ __global__ __launch_bounds__(kThreads, NS == 2 ? 2 : 1) void attention_prefill_k
 #pragma unroll
     for (int st = 0; st < KST; ++st)
       asm volatile("" : : "v"(qf[qt][st].x), "v"(qf[qt][st].y), "v"(qf[qt][st].z), "v"(qf[qt][st].w));
-  for (int ib = 0; ib < nblocks; ++ib) {
-    if (NS == 3 && ib + 1 < nblocks) wait_vmcnt<8>();
+  for (int it = 0; it < niter; ++it) {
+    if (NS == 3 && it + 1 < niter) wait_vmcnt<PW>();
     else wait_vmcnt<0>();
-    barrier_lds();  // block ib landed for every wave; block ib-1 fully consumed
-    if (ib + NS - 1 < nblocks) issue((ib + NS - 1) * 64, (ib + NS - 1) % NS);
-    const int kb = ib * 64;
+    barrier_lds();  // stage it landed for every wave; stage it - 1 fully consumed
+    if (it + NS - 1 < niter) issue(it + NS - 1, (it + NS - 1) % NS);
+    const int kb = 64 * (KS * it + ks);
+    if (KS > 1 && kb >= t) continue;  // wave-uniform: an odd last block is the first share's
     if (CAUSAL && (kb >= s_len || kb > wq0 + 16 * QT - 1)) continue;  // wave-uniform: no query of the wave sees it
-    const uint8_t* st_base = smem + (ib % NS) * STAGE;
+    const uint8_t* st_base = smem + (it % NS) * STAGE + ks * KB;
 
     // Every K fragment of the block is read before the first S MFMA, and every
     // V^T fragment right after the last one, so that these LDS reads are in
@@ -670,7 +766,8 @@ __global__ __launch_bounds__(kThreads, NS == 2 ? 2 : 1) void attention_prefill_k
       const int tq0 = wq0 + 16 * qt;  // first query of the tile
       const bool masked = CAUSAL ? (kb + 63 > tq0 || kb + 63 >= t) : kb + 63 >= t;
       const int lim = (CAUSAL ? min(tq0 + r16, t - 1) : t - 1) - kb - 8 * g;
-      const float alpha = softmax_block(sc[qt], masked, lim, c2, m[qt], den[qt], pf[qt]);
+      const float alpha = CAUSAL ? softmax_block(sc[qt], masked, lim, c2, m[qt], den[qt], pf[qt])
+                                 : softmax_block_free(sc[qt], masked, lim, c2, m[qt], den[qt], pf[qt]);
       rescale<DTN>(o[qt], alpha);
     }
 #pragma unroll
@@ -681,6 +778,33 @@ __global__ __launch_bounds__(kThreads, NS == 2 ? 2 : 1) void attention_prefill_k
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) o[qt][dt] = mfma_bf16(vf[c][dt], pf[qt][c], o[qt][dt]);
       }
+  }
+  // The key shares of one query set are merged through LDS, lane by lane, in the
+  // frame of the larger reference.
+  if constexpr (KS == 2) {
+    static_assert(NW * QT * (DTN + 1) * 1024 <= NS * STAGE, "the shares' sums fit the stages");
+    uint8_t* buf = smem + wave * (QT * (DTN + 1) * 1024) + 16 * lane;
+    barrier_lds();  // every wave is done reading the stages
+    if (ks == 1) {
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+        for (int dt = 0; dt < DTN; ++dt) *reinterpret_cast<f32x4*>(buf + (qt * (DTN + 1) + dt) * 1024) = o[qt][dt];
+        *reinterpret_cast<f32x4*>(buf + (qt * (DTN + 1) + DTN) * 1024) = f32x4{m[qt], den[qt], 0.f, 0.f};
+      }
+    }
+    barrier_lds();
+    if (ks == 1) return;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const f32x4 md = *reinterpret_cast<const f32x4*>(buf + (qt * (DTN + 1) + DTN) * 1024);
+      const float mx = fmaxf(m[qt], md[0]);  // share 0 holds key block 0, so it is a score
+      const float a0 = __builtin_amdgcn_exp2f((m[qt] - mx) * c2), a1 = __builtin_amdgcn_exp2f((md[0] - mx) * c2);
+      den[qt] = den[qt] * a0 + md[1] * a1;
+#pragma unroll
+      for (int dt = 0; dt < DTN; ++dt)
+        o[qt][dt] = o[qt][dt] * a0 + *reinterpret_cast<const f32x4*>(buf + (qt * (DTN + 1) + dt) * 1024) * a1;
+    }
   }
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -854,22 +978,31 @@ extern "C" int ff_attention_full(const void* q, const void* k, const void* vt, v
   FF_REQUIRE(ff_aligned(q, 16) && ff_aligned(k, 16) && ff_aligned(vt, 16) && ff_aligned(y, 8),
              "ff_attention_full: alignment");
   const float c2 = (float)((double)scale * 1.4426950408889634);  // scale * log2(e)
-  // One query tile per wave while that grid fits two workgroups per CU (512;
-  // the 8B tower at 2048 patches, 16 heads: 512 workgroups, tower step 5.97
-  // -> 5.87 ms against two tiles at 256, same bits), else two.
-  // ff_set_tuning(FF_TUNE_ATTN_QT, 1 | 2) overrides the query tiles per wave.
+  // 4 waves x 16 queries while that grid is at most one workgroup per CU (16 heads
+  // at 1024 patches: 15.0 us; two query tiles a wave 20.1). Past that 4 x 32 queries
+  // with the key blocks dealt to two sets of four waves while that is at most one
+  // workgroup per CU: every fragment read from LDS feeds two MFMAs, two waves per
+  // SIMD overlap, and a CU stages the keys once (2048 patches: 34.5 us, 4 x 16
+  // queries at two workgroups per CU 36.0; 41.0 before the narrower stages and
+  // softmax_block_free). Else 4 x 32 queries at two workgroups
+  // per CU. ff_set_tuning(FF_TUNE_ATTN_QT, 1 | 2) forces the query tiles per wave.
   const int qt_env = ff_tuning(FF_TUNE_ATTN_QT);
-  const int qt = qt_env == 1 || qt_env == 2 ? qt_env : ((t + 63) / 64 * heads <= 512 ? 1 : 2);
-  const int qb = 16 * qt * 4;  // one head per workgroup: 4 waves x QT tiles of 16 queries
+  const int64_t w64 = (t + 63) / 64 * heads, w128 = (t + 127) / 128 * heads;
+  const int qt = qt_env == 1 || qt_env == 2 ? qt_env : (w64 <= 256 ? 1 : 2);
+  const int ks = qt == 2 && w64 > 256 && w128 <= 256 ? 2 : 1;
+  constexpr int nw = 4;
+  const int qb = 16 * qt * nw;  // one head per workgroup: nw waves x QT tiles of 16 queries
   const int nqb = (int)((t + qb - 1) / qb);
-  const dim3 grid((unsigned)(nqb * heads)), block(kThreads);
+  const dim3 grid((unsigned)(nqb * heads)), block((unsigned)(64 * nw * ks));
   hipStream_t st = (hipStream_t)stream;
-#define FF_FULL(QT, DO)                                                                                    \
-  if (qt == QT && d_out == DO)                                                                             \
-    hipLaunchKernelGGL((attention_prefill_kernel<QT, 1, 2, false, DO>), grid, block, 0, st, (const bf16_t*)q, \
-                       (const bf16_t*)k, (const bf16_t*)vt, (bf16_t*)y, (int)t, (int)t, (int)t_pad, (int)heads, \
-                       (int)heads, c2, nqb, 0.f);
-  FF_FULL(1, 64) FF_FULL(2, 64) FF_FULL(1, 72) FF_FULL(2, 72) FF_FULL(1, 128) FF_FULL(2, 128)
+#define FF_FULL(QT, DO, KS)                                                                                   \
+  if (qt == QT && d_out == DO && ks == KS)                                                            \
+    hipLaunchKernelGGL((attention_prefill_kernel<QT, 1, 2, false, DO, false, nw, KS>), grid, block, 0, st,        \
+                       (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)vt, (bf16_t*)y, (int)t, (int)t,         \
+                       (int)t_pad, (int)heads, (int)heads, c2, nqb, 0.f);
+#define FF_FULL_D(QT, KS) FF_FULL(QT, 64, KS) FF_FULL(QT, 72, KS) FF_FULL(QT, 128, KS)
+  FF_FULL_D(1, 1) FF_FULL_D(2, 1) FF_FULL_D(2, 2)
+#undef FF_FULL_D
 #undef FF_FULL
   FF_LAUNCH_CHECK("ff_attention_full");
   return FF_OK;

@@ -457,6 +457,39 @@ def test_attention_full(gpu, n, nh, hd):
     assert torch.equal(y2, y)
 
 
+# 16 heads: 64 queries a workgroup (1000 tokens, one per CU), and past that the key
+# blocks dealt to two sets of waves: an odd and an even number of 64-key blocks,
+# ragged and full last blocks, each head width
+@pytest.mark.parametrize("n,hd", [(1000, 72), (1025, 72), (1088, 64), (1100, 128), (1152, 72)])
+@pytest.mark.parametrize("ramp", [0.0, 40.0, float("-inf")])
+def test_attention_full_key_split(gpu, n, hd, ramp):
+    """ff_attention_full against the oracle where its grid splits the keys; with
+    ``ramp`` the scores grow along the keys (by about 4 ramp in natural units), so
+    that the running reference moves many times and the two sets' references
+    differ; with -inf the first two key blocks' scores are -inf (weight 0)."""
+    from fastforward_amd._lib import call, ptr, stream
+    nh = 16
+    q, k, v = (torch.randn(n, nh, hd, generator=_g(50 + i)) for i in range(3))
+    q[:, :, 0] = 4.0
+    k[:, :, 0] = 0
+    if ramp > 0:
+        k[:, :, 0] = torch.linspace(0, ramp, n)[:, None] * hd ** 0.5 / 4
+    elif ramp < 0:
+        k[:128, :, 0] = ramp
+    q, k, v = (t.to(BF16) for t in (q, k, v))
+    n_pad = (n + 63) // 64 * 64
+    qd, kd = (torch.zeros(nh, n, 128, dtype=BF16, device=DEV) for _ in range(2))
+    qd[:, :, :hd], kd[:, :, :hd] = q.transpose(0, 1).to(DEV), k.transpose(0, 1).to(DEV)
+    vt = torch.zeros(nh, 128, n_pad, dtype=BF16, device=DEV)
+    vt[:, :hd, :n] = v.permute(1, 2, 0).to(DEV)
+    y = torch.full((n, nh * hd), float("nan"), device=DEV, dtype=BF16)
+    call("ff_attention_full", ptr(qd), ptr(kd), ptr(vt), ptr(y), n, n_pad, nh, hd, float(hd ** -0.5), stream())
+    got, want = y.cpu().float(), OV.attention(q, k, v, hd ** -0.5).float()
+    # bf16(p) and the bf16 output: 2^-9 each relative to the weights' mean of |v|
+    assert float((got - want).norm() / want.norm()) <= 5e-3
+    assert float((got - want).abs().max()) <= (1 / 16 if ramp > 0 else 1 / 64)   # |v| up to 4 with one key dominating
+
+
 def test_pos_interp_bit_exact(gpu):
     from fastforward_amd.vision import VisionConfig, interp_taps
     from fastforward_amd._lib import call, ptr, stream
