@@ -123,6 +123,30 @@ def _packed_gemm(op, q, s, s_rows, sw, sw_cols, y):
     return y
 
 
+ROWS_MAX_CODES = 49152  # FF_LINEAR_FP8_ROWS_MAX
+
+
+def rows_fit(op, m):
+    """Whether ``m`` rows of ``op`` run as one launch (``linear_rows``): the op keeps
+    only its packed codes, so that the single-row kernel is the one its product
+    takes anyway, and the rows' codes fit the kernel's LDS."""
+    return m <= 4 and m * op.weight.shape[1] <= ROWS_MAX_CODES and isinstance(op.weight, PackedCodes) and m > 0
+
+
+def linear_rows(op, x, y):
+    """y = op(x) for at most four rows (``rows_fit``), quantised inside the product's
+    launch: the same bits as the quantiser and the GEMM."""
+    m, k = x.shape
+    n = op.weight.shape[0]
+    if isinstance(op, StaticFP8Linear):
+        call("ff_linear_fp8_rows", ptr(x), x.stride(0), ptr(op.input_scale), float(op.inverse_scale), ptr(op.packed),
+             ptr(op.weight_scale), 0, ptr(y), y.stride(0), m, n, k, stream())
+    else:
+        call("ff_linear_fp8_rows", ptr(x), x.stride(0), None, 0.0, ptr(op.packed), ptr(op.scale), 1, ptr(y),
+             y.stride(0), m, n, k, stream())
+    return y
+
+
 class FP8Linear:
     """Per-channel e4m3 weights + per-token dynamic activation quant
     (_legacy/fp8_private.py:21-38). ``scale`` is (1, N) fp32 as in the reference.
@@ -185,8 +209,15 @@ class FP8Linear:
 
     def __call__(self, x):
         assert x.is_cuda and x.dtype == BF16
+        n, k = self.weight.shape
+        if 0 < x.numel() <= 4 * k and x.shape[-1] == k and rows_fit(self, x.numel() // k):
+            flat = _rows(x)
+            if flat.stride(-1) != 1:
+                flat = flat.contiguous()
+            y = linear_rows(self, flat, torch.empty((flat.shape[0], n), device=x.device, dtype=BF16))
+            return y if x.dim() == 2 else y.reshape(*x.shape[:-1], n)
         q, s = self.quantize(x)
-        return self.gemm(q, s).reshape(*x.shape[:-1], self.weight.shape[0])
+        return self.gemm(q, s).reshape(*x.shape[:-1], n)
 
 
 class StaticFP8Linear:
@@ -225,6 +256,8 @@ class StaticFP8Linear:
             flat = flat.contiguous()
         m, k = flat.shape
         n = self.weight.shape[0]
+        if k == self.weight.shape[1] and x.dtype == BF16 and rows_fit(self, m):
+            return linear_rows(self, flat, torch.empty((m, n), device=x.device, dtype=BF16))
         q = torch.empty((m, k), device=x.device, dtype=E4M3)
         call("ff_quant_static_fp8", ptr(flat), ptr(q), m, m, k, float(self.inverse_scale), stream())
         y = torch.empty((m, n), device=x.device, dtype=BF16)

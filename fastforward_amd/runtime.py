@@ -26,7 +26,7 @@ import torch
 
 from . import ops
 from ._lib import call, ptr, stream
-from .linear import FP8Linear, Int4, Linear, StaticFP8Linear, gemm_pk_workspace
+from .linear import FP8Linear, Int4, Linear, StaticFP8Linear, gemm_pk_workspace, linear_rows, rows_fit
 
 BF16 = torch.bfloat16
 E4M3 = torch.float8_e4m3fn
@@ -347,11 +347,20 @@ class Runtime:
         lw = L[-1]
         h = self.h[cur]
         self._attention_fused(lw, s, tail=True)
-        self._gemm(self.aq, self.as_, lw.o, self.o, 1, s)
+        if rows_fit(lw.o, 1):
+            linear_rows(lw.o, self.attn[:1], self.o[:1])
+        else:
+            call("ff_quant_rows_fp8", ptr(self.attn), HQ * D, ptr(self.aq), ptr(self.as_), 1, HQ * D, s)
+            self._gemm(self.aq, self.as_, lw.o, self.o, 1, s)
         call("ff_gather_rows", ptr(h), H, ptr(self.pick), ptr(self.hp), H, 1, H, T, s)
         call("ff_add_rms_quant", ptr(self.hp), ptr(self.o), None, ptr(lw.post_norm.weight), ptr(self.res), None,
              ptr(self.pq), ptr(self.ps), 1, H, float(lw.post_norm.variance_epsilon), 0, 0, s)
-        self._mlp_fused(lw, self.pq, self.ps, 1, self.dn, s)
+        fit = rows_fit(lw.down, 1)
+        self._gateup_fused(lw, self.pq, self.ps, 1, s, quant=not fit)
+        if fit:
+            linear_rows(lw.down, self.hm[:1], self.dn[:1])
+        else:
+            self._gemm(self.mq, self.ms, lw.down, self.dn, 1, s)
         call("ff_lm_readout", ptr(self.res), ptr(self.dn), ptr(w.norm.weight), ptr(w.head), ptr(self.logits), H,
              w.head.shape[0], float(w.norm.variance_epsilon), s)
         return self.logits
@@ -368,7 +377,6 @@ class Runtime:
         if tail:
             call("ff_attention_vt", ptr(self.yq), ptr(self.yk), ptr(self.vt), ptr(self.pick), 1, ptr(self.attn),
                  1, T, Tp, HQ, HK, D, float(cfg.scaling), s)
-            call("ff_quant_rows_fp8", ptr(self.attn), HQ * D, ptr(self.aq), ptr(self.as_), 1, HQ * D, s)
         else:
             call("ff_attention_vt", ptr(self.yq), ptr(self.yk), ptr(self.vt), None, 0, ptr(self.attn), T, T, Tp,
                  HQ, HK, D, float(cfg.scaling), s)
@@ -382,16 +390,13 @@ class Runtime:
         call("ff_gemm_fp8_pk", ptr(q), ptr(sc), 1, ptr(op.weight), ptr(op.packed), ptr(op.scale), 1, ptr(out), n,
              m, n, k, ptr(self.gws), self.gws.numel(), s)
 
-    def _gateup_fused(self, lw, q, sc, m, s):
+    def _gateup_fused(self, lw, q, sc, m, s, quant=True):
         I, H = self.cfg.inter, self.cfg.hidden
-        # gate/up GEMM with SwiGLU in its epilogue, then per-token quant from its row maxima
+        # gate/up GEMM with SwiGLU in its epilogue, then (quant) per-token quant from its row maxima
         call("ff_gemm_fp8_swiglu_pk", ptr(q), ptr(sc), ptr(lw.gateup.weight), ptr(lw.gateup.packed),
              ptr(lw.gateup.scale), ptr(self.hm), I, ptr(self.pmax), m, I, H, s)
-        call("ff_quant_rows_pmax", ptr(self.hm), I, ptr(self.pmax), I // 64, ptr(self.mq), ptr(self.ms), m, I, s)
-
-    def _mlp_fused(self, lw, q, sc, m, out, s):
-        self._gateup_fused(lw, q, sc, m, s)
-        self._gemm(self.mq, self.ms, lw.down, out, m, s)
+        if quant:
+            call("ff_quant_rows_pmax", ptr(self.hm), I, ptr(self.pmax), I // 64, ptr(self.mq), ptr(self.ms), m, I, s)
 
     def _step_static(self, trace=None):
         """The fused step for static-scale linears (the reference's calibrated
@@ -438,8 +443,11 @@ class Runtime:
         self._qkv_static(lw, T, s)
         call("ff_attention_vt", ptr(self.yq), ptr(self.yk), ptr(self.vt), ptr(self.pick), 1, ptr(self.attn), 1, T,
              Tp, HQ, HK, D, float(cfg.scaling), s)
-        call("ff_quant_static_fp8", ptr(self.attn), ptr(self.aq), 1, 1, HQ * D, float(lw.o.inverse_scale), s)
-        self._gemm_static(self.aq, lw.o, self.o, 1, s)
+        if rows_fit(lw.o, 1):
+            linear_rows(lw.o, self.attn, self.o[:1])
+        else:
+            call("ff_quant_static_fp8", ptr(self.attn), ptr(self.aq), 1, 1, HQ * D, float(lw.o.inverse_scale), s)
+            self._gemm_static(self.aq, lw.o, self.o, 1, s)
         call("ff_gather_rows", ptr(h), H, ptr(self.pick), ptr(self.hp), H, 1, H, T, s)
         call("ff_add_rms_quant_static", ptr(self.hp), ptr(self.o), None, ptr(lw.post_norm.weight), ptr(self.res), None,
              ptr(self.pq), float(lw.gateup.inverse_scale), 1, H, float(lw.post_norm.variance_epsilon), 0, 0, s)

@@ -224,6 +224,18 @@ int ff_gemm_fp8_pk(const void* qa, const float* sa, int sa_rows, const void* qw,
                    const float* sw, int sw_cols, void* y, int64_t ldy, int64_t m, int64_t n, int64_t k,
                    void* workspace, int64_t workspace_bytes, ff_stream_t stream);
 
+/* A whole FP8 linear of at most four rows in one launch: x (m, k) bf16 (row
+ * stride x_rs) quantised inside the kernel, per token as ff_quant_rows_fp8 (sa
+ * NULL) or as ff_quant_static_fp8 with the multiplier inv and the scale sa[0], then
+ * the single-row kernel of ff_gemm_fp8_pk on the packed copy (qw NULL there): the
+ * same bits as those two calls. m 1..4, n % 16 == 0, k % 128 == 0, k >= 512, m * k
+ * <= FF_LINEAR_FP8_ROWS_MAX (the codes' LDS). Replaces Linear.apply of the
+ * pick-only tail (_family/night_runtime.py:92-105, _legacy/fp8_private.py:33-38). */
+#define FF_LINEAR_FP8_ROWS_MAX 49152
+int ff_linear_fp8_rows(const void* x, int64_t x_rs, const float* sa, float inv, const void* qw_packed,
+                       const float* sw, int sw_cols, void* y, int64_t ldy, int64_t m, int64_t n, int64_t k,
+                       ff_stream_t stream);
+
 /* Down projection + the next add_rms (no reference counterpart as one op: the
  * down Linear of scaled_qwen_runtime.py:35-39 followed by the add_rms of
  * _legacy/lower_kernels.py:7-32 with the per-token quant of

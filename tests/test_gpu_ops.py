@@ -939,6 +939,42 @@ def test_fp8linear_keeps_one_copy(gpu, m, k, n):
     _assert_fp8_gemm(y1.cpu(), qa, sa, qw, sw, O.fp8_gemm(qa, sa, qw, sw), f"one-copy FP8Linear {m}x{k}x{n}")
 
 
+# the smallest k and n of the packed layout, ragged numbers of k steps per wave, the
+# limits of the codes' LDS (49152 bytes) and past it
+@pytest.mark.parametrize("m,k,n", [(1, 512, 128), (4, 512, 128), (2, 2560, 256), (3, 9728, 128), (4, 12288, 256),
+                                   (1, 25600, 128), (2, 25600, 128), (1, 49152, 128)])
+@pytest.mark.parametrize("static", [False, True])
+def test_linear_rows_equals_quantise_and_gemm(gpu, m, k, n, static):
+    """A linear of at most four rows quantises inside the product's launch
+    (ff_linear_fp8_rows, up to 49152 codes): bit for bit the quantiser and the GEMM
+    as two calls, for rows of ordinary values, zeros, one infinity and one NaN, and
+    for a strided view."""
+    from fastforward_amd.linear import FP8Linear, StaticFP8Linear, _packed_gemm, rows_fit
+    w = (torch.randn(n, k, generator=_g(190)) * 0.02).to(BF16).to(DEV)
+    op = StaticFP8Linear(w, 56.0) if static else FP8Linear(w)
+    assert rows_fit(op, m) == (m * k <= 49152)
+    wide = torch.randn(m, k + 8, generator=_g(191)).to(BF16)
+    special = wide.clone()
+    special[0] = 0
+    special[-1, 3] = float("inf")
+    if m > 1:
+        special[1, 5] = float("nan")
+    for x in (wide[:, :k], wide[:, :k].contiguous(), special[:, :k].contiguous()):
+        x = x.to(DEV) if x.is_contiguous() else wide.to(DEV)[:, :k]
+        got = op(x)
+        ref = torch.empty(m, n, device=DEV, dtype=BF16)
+        if static:
+            q = torch.empty(m, k, device=DEV, dtype=torch.float8_e4m3fn)
+            from fastforward_amd._lib import call, ptr, stream
+            xc = x.contiguous()
+            call("ff_quant_static_fp8", ptr(xc), ptr(q), m, m, k, float(op.inverse_scale), stream())
+            _packed_gemm(op, q, op.input_scale, 0, op.weight_scale, 0, ref)
+        else:
+            op.gemm(*op.quantize(x), out=ref)
+        assert got.shape == (m, n)
+        assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
 @pytest.mark.parametrize("m,i,k", [(1, 12288, 4096), (3, 6144, 2048), (4, 640, 512), (20, 6144, 2048)])
 def test_swiglu_single_copy_rows(gpu, m, i, k):
     """The gate/up + SwiGLU launch on the packed copy alone (qw NULL): for m <= 4
