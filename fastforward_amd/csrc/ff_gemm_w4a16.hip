@@ -600,7 +600,7 @@ __device__ __forceinline__ void w4pk_mainloop(f32x4 (&acc)[BM / 16][CW / 16], ui
   constexpr int HALF = BM * 128;  // one 128-byte half of every row of a stage
   constexpr int STAGE = 2 * HALF;
   static_assert(A_CHUNKS >= kThreads, "at least one full activation round");
-  static_assert(RA >= 9, "a group's MFMAs carry the next group's 7 dequantisation pieces, 2 MFMAs before its use");
+  static_assert(RA >= 6, "a group's MFMAs carry the next group's 7 dequantisation pieces, 2 MFMAs before its use");
   const int tid = threadIdx.x, lane = tid & 63;
   const int r16 = lane & 15, g = lane >> 4;
   const int kend = kt0 + nk;
@@ -739,7 +739,10 @@ __device__ __forceinline__ void w4pk_mainloop(f32x4 (&acc)[BM / 16][CW / 16], ui
         static_for<0, RA>([&](auto I_) {
           constexpr int i = decltype(I_)::value;
           mfma_bf16_acc(acc[i][j], bcur, a[sub & 1][i]);
-          if constexpr (i < 7) d.template piece<i>();
+          // the 7 pieces over the group's first RA - 2 MFMAs: one each at 9, fewer rows two
+          constexpr int p0 = i < RA - 2 ? (RA >= 9 ? (i < 7 ? i : 7) : i * 7 / (RA - 2)) : 7;
+          constexpr int p1 = i < RA - 2 ? (RA >= 9 ? (i < 7 ? i + 1 : 7) : (i + 1) * 7 / (RA - 2)) : 7;
+          static_for<p0, p1>([&](auto P_) { d.template piece<decltype(P_)::value>(); });
           if constexpr (in_step && jn == 0) readA(st, subn, i, a[subn & 1][i]);
           if constexpr (!in_step) readA(stn, 0, i, a[0][i]);  // substep 3 runs on a[1]
           // The step's memory work, one instruction group per MFMA slot: the
@@ -1021,15 +1024,25 @@ bool w4pk_gemv_fits(int64_t m, int64_t n, int64_t k, int64_t group) {
 }
 
 // Plans of the packed path. Plain: 144 x 384 tiles (CW 96) when they fill the
-// GPU unsplit; otherwise 144 x 256 tiles (CW 64) with k split until about one
+// GPU unsplit; otherwise BM x 256 tiles (CW 64) with k split until about one
 // workgroup per CU (at most 8 ways, at least one pair of k steps each). SwiGLU:
-// 144 x (192 gate + 192 up) tiles when the channels divide, else 144 x (128 +
+// BM x (192 gate + 192 up) tiles when the channels divide, else BM x (128 +
 // 128). Shapes outside the packed path's limits are reported as not fitting.
+//
+// BM: a wave dequantises its weights once for its BM rows, so tall tiles spend the
+// least dequantisation per product, but the rows past m are wasted. A step costs
+// about BM + 16 rows' time down to 96 rows, where the dequantisation takes as long
+// as the MFMAs. What the choice gives over 144 rows throughout (weights streamed):
+// gate/up of 176 tokens 2560 -> 2 x 9728 (group 32) 46.6 -> 37.7 us, 4096 -> 2 x
+// 12288 91.8 -> 73.7; 320 tokens 2048 -> 2 x 6144 49.4 -> 39.6; down of 176 tokens
+// 12288 -> 4096 42.7 -> 34.0; 576 tokens keep 144.
 constexpr int kW4BM = 144;
+constexpr int kW4Rows[4] = {144, 128, 112, 96};
 
 struct W4PkPlan {
   int cw = 0;      // 0: the packed path does not take this shape
   int splits = 1;
+  int bm = kW4BM;
 };
 
 bool w4pk_common_fits(int64_t m, int64_t k, int64_t group) {
@@ -1054,12 +1067,22 @@ W4PkPlan w4pk_plan(int64_t m, int64_t n, int64_t k, int64_t group) {
     return p;
   }
   if (n % 256) return p;
-  const int64_t tiles = tm * (n / 256), pairs = k / (2 * kPkStep);
-  int64_t s = 1;
-  if (const int f = ff_tuning(FF_TUNE_W4A16_SPLITS)) s = f;
-  else if (tiles < 192) s = 256 / tiles;
-  p.cw = 64;
-  p.splits = (int)std::max<int64_t>(1, std::min<int64_t>({s, 8, pairs}));
+  const int64_t pairs = k / (2 * kPkStep);
+  int64_t best = 0;
+  for (const int bm : kW4Rows) {
+    const int64_t tiles = (m + bm - 1) / bm * (n / 256);
+    int64_t s = 1;
+    if (const int f = ff_tuning(FF_TUNE_W4A16_SPLITS)) s = f;
+    else if (tiles < 192) s = 256 / tiles;
+    s = std::max<int64_t>(1, std::min<int64_t>({s, 8, pairs}));
+    const int64_t cost = (tiles * s + 255) / 256 * ((pairs + s - 1) / s) * (bm + 16);
+    if (p.cw == 0 || cost < best) {
+      p.cw = 64;
+      p.splits = (int)s;
+      p.bm = bm;
+      best = cost;
+    }
+  }
   return p;
 }
 
@@ -1075,17 +1098,19 @@ int w4pk_swiglu_cw(int64_t m, int64_t i, int64_t k, int64_t group) {
 int64_t w4pk_workspace(int64_t m, int64_t n, int64_t k, int64_t group) {
   const W4PkPlan p = w4pk_plan(m, n, k, group);
   if (p.cw == 0 || p.splits <= 1) return 0;
-  return (m + kW4BM - 1) / kW4BM * (n / (4 * p.cw)) * p.splits * kW4BM * 4 * p.cw * 4;
+  return (m + p.bm - 1) / p.bm * (n / (4 * p.cw)) * p.splits * p.bm * 4 * p.cw * 4;
 }
 
-// Row-tile height of the packed SwiGLU GEMM with 96-channel wave tiles: 160
-// where it keeps the grid in one round of 256 workgroups that 144 would spill
-// into a second (the 8B gate/up at 577..640 and 1153..1280 tokens), counted as
-// rounds x (BM + 16) rows per CU; 144 otherwise. 160 rows is the most the
-// accumulators fit (240 of 256 AGPRs), and the main loop needs at least 144.
-int w4_swiglu_bm(int64_t m, int64_t tiles_n) {
+// Row-tile height of the packed SwiGLU GEMM: the fewest rounds of 256 workgroups x
+// (BM + 16) rows per CU, the tallest among equals. With 96-channel wave tiles 160
+// rows are the most the accumulators fit (240 of 256 AGPRs): the 8B gate/up at
+// 577..640 and 1153..1280 tokens keeps its rounds with them.
+int w4_swiglu_bm(int64_t m, int64_t tiles_n, int cw) {
   const auto cost = [&](int bm) { return ((m + bm - 1) / bm * tiles_n + 255) / 256 * (bm + 16); };
-  return cost(160) < cost(kW4BM) ? 160 : kW4BM;
+  int best = kW4BM;
+  for (const int bm : kW4Rows)
+    if (cost(bm) < cost(best)) best = bm;
+  return cw == 96 && cost(160) < cost(best) ? 160 : best;
 }
 
 template <int CW, bool SWIGLU, int BM = kW4BM>
@@ -1102,6 +1127,16 @@ void launch_w4pk(const void* x, int64_t ldx, const void* frag, const void* fscal
     hipLaunchKernelGGL(w4pk_reduce_kernel, dim3((unsigned)((chunks + kThreads - 1) / kThreads)), dim3(kThreads), 0, s,
                        (const float*)ws, splits, (int64_t)tiles_m * BM, (bf16_t*)y, ldy, m, n);
   }
+}
+
+// launch_w4pk at the run-time row-tile height bm (one of kW4Rows).
+template <int CW, bool SWIGLU>
+void launch_w4pk_rows(int bm, const void* x, int64_t ldx, const void* frag, const void* fscales, int gshift, void* y,
+                      int64_t ldy, int m, int n, int k, int splits, void* ws, hipStream_t s) {
+  if (bm == 96) launch_w4pk<CW, SWIGLU, 96>(x, ldx, frag, fscales, gshift, y, ldy, m, n, k, splits, ws, s);
+  else if (bm == 112) launch_w4pk<CW, SWIGLU, 112>(x, ldx, frag, fscales, gshift, y, ldy, m, n, k, splits, ws, s);
+  else if (bm == 128) launch_w4pk<CW, SWIGLU, 128>(x, ldx, frag, fscales, gshift, y, ldy, m, n, k, splits, ws, s);
+  else launch_w4pk<CW, SWIGLU>(x, ldx, frag, fscales, gshift, y, ldy, m, n, k, splits, ws, s);
 }
 
 }  // namespace
@@ -1168,11 +1203,11 @@ int gemm_w4a16_pk_partials(const void* x, int64_t ldx, const void* frag, const v
   const int64_t need = w4pk_workspace(m, n, k, group);
   FF_REQUIRE(workspace && workspace_bytes >= need && ff_aligned(workspace, 16),
              "ff_gemm_w4a16_pk: workspace of %lld bytes (16-byte aligned) required", (long long)need);
-  launch_w4pk<64, false>(x, ldx, frag, frag_scales, w4_gshift(group), nullptr, 0, (int)m, (int)n, (int)k, p.splits,
-                         workspace, st);
+  launch_w4pk_rows<64, false>(p.bm, x, ldx, frag, frag_scales, w4_gshift(group), nullptr, 0, (int)m, (int)n, (int)k,
+                              p.splits, workspace, st);
   FF_LAUNCH_CHECK("ff_gemm_w4a16_pk");
   *splits = p.splits;
-  *mp = (m + kW4BM - 1) / kW4BM * kW4BM;
+  *mp = (m + p.bm - 1) / p.bm * p.bm;
   return FF_OK;
 }
 }  // namespace ff
@@ -1201,7 +1236,8 @@ extern "C" int ff_gemm_w4a16_pk(const void* x, int64_t ldx, const void* packed, 
   if (p.cw == 96)
     launch_w4pk<96, false>(x, ldx, frag, frag_scales, gs, y, ldy, (int)m, (int)n, (int)k, 1, nullptr, s);
   else
-    launch_w4pk<64, false>(x, ldx, frag, frag_scales, gs, y, ldy, (int)m, (int)n, (int)k, p.splits, workspace, s);
+    launch_w4pk_rows<64, false>(p.bm, x, ldx, frag, frag_scales, gs, y, ldy, (int)m, (int)n, (int)k, p.splits,
+                                workspace, s);
   FF_LAUNCH_CHECK("ff_gemm_w4a16_pk");
   return FF_OK;
 }
@@ -1229,19 +1265,21 @@ extern "C" int ff_gemm_w4a16_swiglu_pk(const void* x, int64_t ldx, const void* f
   const int gs = w4_gshift(group);
   if (gemv)
     launch_gemv_w4pk<true>(x, ldx, frag, frag_scales, gs, h, ldh, (int)m, (int)(2 * i), (int)k, s);
-  else if (cw == 96 && w4_swiglu_bm(m, 2 * i / 384) == 160)
+  else if (cw == 96 && w4_swiglu_bm(m, 2 * i / 384, 96) == 160)
     launch_w4pk<96, true, 160>(x, ldx, frag, frag_scales, gs, h, ldh, (int)m, (int)(2 * i), (int)k, 1, nullptr, s);
   else if (cw == 96)
-    launch_w4pk<96, true>(x, ldx, frag, frag_scales, gs, h, ldh, (int)m, (int)(2 * i), (int)k, 1, nullptr, s);
+    launch_w4pk_rows<96, true>(w4_swiglu_bm(m, 2 * i / 384, 96), x, ldx, frag, frag_scales, gs, h, ldh, (int)m,
+                               (int)(2 * i), (int)k, 1, nullptr, s);
   else
-    launch_w4pk<64, true>(x, ldx, frag, frag_scales, gs, h, ldh, (int)m, (int)(2 * i), (int)k, 1, nullptr, s);
+    launch_w4pk_rows<64, true>(w4_swiglu_bm(m, 2 * i / 256, 64), x, ldx, frag, frag_scales, gs, h, ldh, (int)m,
+                               (int)(2 * i), (int)k, 1, nullptr, s);
   FF_LAUNCH_CHECK("ff_gemm_w4a16_swiglu_pk");
   return FF_OK;
 }
 
 // ------------------------------------------------------------------ fused QKV
 //
-// ff_gemm_w4a16_qkv: the packed GEMM of the QKV weight on 144 x 256 tiles (two
+// ff_gemm_w4a16_qkv: the packed GEMM of the QKV weight on BM x 256 tiles (two
 // heads of 128 per tile), its fp32 partials always going to the workspace, then
 // w4pk_qkv_kernel per (tile, 16-token group): the partials added in split
 // order and rounded to bf16 (the values of ff_gemm_w4a16_pk), staged in LDS,
@@ -1328,13 +1366,12 @@ __global__ __launch_bounds__(kThreads) void vt_zero_tail_kernel(bf16_t* __restri
     vt[(i / (t_pad - t0)) * t_pad + t0 + i % (t_pad - t0)] = 0;
 }
 
-// Splits of the QKV GEMM: the 144 x 256 tiles of w4pk_plan, k split until
-// about one workgroup per CU.
-int w4pk_qkv_splits(int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = (m + kW4BM - 1) / kW4BM * (n / 256), pairs = k / (2 * kPkStep);
-  int64_t s = tiles >= 192 ? 1 : 256 / tiles;
-  if (const int f = ff_tuning(FF_TUNE_W4A16_SPLITS)) s = f;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({s, 8, pairs}));
+// Row-tile height and splits of the QKV GEMM: those of w4pk_plan (the same sums as
+// the plain product), on 256-column tiles throughout.
+W4PkPlan w4pk_qkv_plan(int64_t m, int64_t n, int64_t k, int64_t group) {
+  W4PkPlan p = w4pk_plan(m, n, k, group);
+  if (p.cw == 96) p.cw = 64;  // unsplit and 144 rows
+  return p;
 }
 
 bool w4pk_qkv_fits(int64_t m, int64_t k, int64_t hq, int64_t hk, int64_t group) {
@@ -1349,9 +1386,8 @@ extern "C" int ff_gemm_w4a16_qkv_workspace(int64_t m, int64_t k, int64_t hq, int
                                            int64_t* bytes) {
   FF_REQUIRE(bytes && m >= 0 && k > 0 && hq > 0 && hk > 0 && group > 0, "ff_gemm_w4a16_qkv_workspace: bad arguments");
   const int64_t n = (hq + 2 * hk) * kHeadDim;
-  *bytes = w4pk_qkv_fits(m, k, hq, hk, group)
-               ? (m + kW4BM - 1) / kW4BM * (n / 256) * w4pk_qkv_splits(m, n, k) * kW4BM * 256 * 4
-               : 0;
+  const W4PkPlan p = w4pk_qkv_plan(m, n, k, group);
+  *bytes = w4pk_qkv_fits(m, k, hq, hk, group) ? (m + p.bm - 1) / p.bm * (n / 256) * p.splits * p.bm * 256 * 4 : 0;
   return FF_OK;
 }
 
@@ -1378,18 +1414,23 @@ extern "C" int ff_gemm_w4a16_qkv(const void* x, int64_t ldx, const void* frag, c
   FF_REQUIRE(workspace && workspace_bytes >= need && ff_aligned(workspace, 16),
              "ff_gemm_w4a16_qkv: workspace of %lld bytes (16-byte aligned) required", (long long)need);
   const int64_t n = (hq + 2 * hk) * kHeadDim;
-  const int splits = w4pk_qkv_splits(m, n, k);
-  const int tiles_m = (int)((m + kW4BM - 1) / kW4BM), tiles_n = (int)(n / 256);
+  const W4PkPlan p = w4pk_qkv_plan(m, n, k, group);
+  const int tiles_m = (int)((m + p.bm - 1) / p.bm), tiles_n = (int)(n / 256);
   const hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL((gemm_w4a16_pk_kernel<kW4BM, 64, false>), dim3((unsigned)(tiles_m * tiles_n * splits)),
-                     dim3(kThreads), 0, s, (const bf16_t*)x, ldx, (const uint8_t*)frag, (const float*)frag_scales,
-                     w4_gshift(group), nullptr, 0, (int)m, (int)n, (int)k, tiles_m, tiles_n, splits,
-                     (f32x4*)workspace);
   const W4Qkv qe{(const bf16_t*)q_norm, (const bf16_t*)k_norm, eps_q, eps_k, (const bf16_t*)cos,
                  (const bf16_t*)sin, (bf16_t*)yq, (bf16_t*)yk, (bf16_t*)vt, (int)hq, (int)hk, (int)t_pad};
-  hipLaunchKernelGGL((w4pk_qkv_kernel<kW4BM>), dim3((unsigned)(tiles_m * tiles_n * (kW4BM / 16))), dim3(kThreads),
-                     0, s, (const f32x4*)workspace, splits, (int)m, tiles_m, qe);
-  const int covered = tiles_m * kW4BM;
+#define FF_QKV(BM)                                                                                               \
+  if (p.bm == BM) {                                                                                              \
+    hipLaunchKernelGGL((gemm_w4a16_pk_kernel<BM, 64, false>), dim3((unsigned)(tiles_m * tiles_n * p.splits)),    \
+                       dim3(kThreads), 0, s, (const bf16_t*)x, ldx, (const uint8_t*)frag,                        \
+                       (const float*)frag_scales, w4_gshift(group), nullptr, 0, (int)m, (int)n, (int)k, tiles_m, \
+                       tiles_n, p.splits, (f32x4*)workspace);                                                    \
+    hipLaunchKernelGGL((w4pk_qkv_kernel<BM>), dim3((unsigned)(tiles_m * tiles_n * (BM / 16))), dim3(kThreads),   \
+                       0, s, (const f32x4*)workspace, p.splits, (int)m, tiles_m, qe);                            \
+  }
+  FF_QKV(96) FF_QKV(112) FF_QKV(128) FF_QKV(144)
+#undef FF_QKV
+  const int covered = tiles_m * p.bm;
   if (t_pad > covered)
     hipLaunchKernelGGL(vt_zero_tail_kernel, dim3(64), dim3(kThreads), 0, s, (bf16_t*)vt, (int)(hk * kHeadDim),
                        (int)t_pad, covered);

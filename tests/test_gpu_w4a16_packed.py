@@ -119,6 +119,30 @@ def test_w4a16_packed_vs_lds_kernel_and_exact(gpu, tuning, m, k, n, sym, group):
     assert float((y - exact).abs().max() / rms) <= 0.05
 
 
+# row tiles of 96, 112, 128 and 144 rows: full, one row short, one row past
+@pytest.mark.parametrize("m", [5, 96, 97, 111, 112, 127, 128, 129, 143, 176, 192, 200, 224, 255, 289])
+@pytest.mark.parametrize("sym,group", [(True, 128), (False, 32)])
+def test_w4a16_packed_row_tiles(gpu, tuning, m, sym, group):
+    """Every row-tile height of the packed kernels at its edges: the plain product
+    with k unsplit equals the LDS-staged kernel bit for bit, the SwiGLU form the
+    unfused op sequence on it, the split product the exact one (as above)."""
+    from fastforward_amd import ops
+    from fastforward_amd.linear import Int4
+    k, n = 1024, 512
+    x = torch.randn(m, k, generator=_g(170)).to(BF16)
+    w = (torch.randn(n, k, generator=_g(171)) * 0.02).to(BF16)
+    op = Int4(w.to(DEV), group=group, symmetric=sym).pack()
+    xd = x.to(DEV)
+    ref = _unsplit_lds(op, xd, tuning)
+    assert op.swiglu_fits(m)
+    assert torch.equal(op.swiglu(xd), ops.swiglu(*ref.chunk(2, -1)))
+    tuning(FF_TUNE_W4A16_SPLITS, 1)
+    assert torch.equal(op(xd), ref)
+    tuning(FF_TUNE_W4A16_SPLITS, 0)
+    exact = x.double() @ O.int4_dequant(op.packed.cpu(), op.scales.cpu(), group).double().T
+    assert float((op(xd).cpu().double() - exact).norm() / exact.norm()) <= 5e-3
+
+
 @pytest.mark.parametrize("n,k", [(256, 256), (256, 512)])
 def test_w4a16_packed_dequant_bit_exact_via_one_hot(gpu, n, k):
     """x = rows of the identity, so y[r, c] = bf16((q-8)*s + z) for k = r exactly,
