@@ -609,7 +609,10 @@ __global__ __launch_bounds__(kThreads, BM <= 96 && !PF ? 2 : 1) void gemm_fp8_sp
   int logical = b;
   if (nblk % kXcds == 0) logical = (b % kXcds) * (nblk / kXcds) + b / kXcds;
   const int tm = logical % tiles_m, rest = logical / tiles_m;  // M fastest: L2 shares weights
-  const int split = rest % S, tn = rest / S;
+  // Splits outermost: an XCD then reads one split's k range of the activations
+  // instead of all of them (8B down, 576 tokens, with its reduction, weights
+  // streamed: 41.1 -> 40.1 us; 32B 1024 x 25600 x 5120, unsplit, unchanged).
+  const int tn = rest % tiles_n, split = rest / tiles_n;
   const int m0 = tm * BM, n0 = tn * BN;
   const int tid = threadIdx.x, wave = tid >> 6;
   // this split's k steps: the kt / U blocks of U steps (U = the main loop's
@@ -809,16 +812,18 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k) {
   }
   if (m <= 256) {
     // Short m (up to four 64-row tiles): 64 x 256 tiles, k split the most ways
-    // among 8, 6, 5, 4 and 2 that keeps the grid within 256 workgroups (8, 4
-    // and 2 where they divide k into whole unrolled blocks; 6 and 5, whose
+    // among 8, 6, 5 and 4 that keeps the grid within 256 workgroups (8 and 4
+    // where they divide k into whole unrolled blocks; 6 and 5, whose
     // split kernels run pk_mainloop_pf and deal out 2-step blocks, where every
     // split gets at least two of them): 176 tokens of the 8B shape, o and down
     // 48 tiles x 5 splits, 240 workgroups (4 splits, 192 workgroups, took the
     // 4.47 ms step to 4.31 ms against small_plan's 64 x 128 tiles for o and
-    // 144 x 256 tiles split 8 ways for down).
+    // 144 x 256 tiles split 8 ways for down). Wider products, which only 2 splits
+    // would fit, run unsplit on small_plan's tiles: 176 x 4096 x 6144 with its
+    // reduction 20.4 us split 2 ways, 18.0 unsplit.
     const int64_t t64 = (m + 63) / 64 * (n / kSpBN);
-    for (const int sp : {8, 6, 5, 4, 2}) {
-      const bool even = sp == 8 || sp == 4 || sp == 2;
+    for (const int sp : {8, 6, 5, 4}) {
+      const bool even = sp == 8 || sp == 4;
       if (t64 * sp <= 256 && (even ? kt % (sp * kSpU) == 0 : kt >= 4 * sp)) return SplitPlan{64, sp};
     }
   }
@@ -869,7 +874,8 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k) {
 struct SmallTile {
   int bm = 0, cw = 0;
 };
-SmallTile small_plan(int64_t m, int64_t n, int64_t k, bool any_count = false) {
+static_assert(lcm3(4, 4, 2) == kSpU, "k % (128 kSpU) == 0 covers the narrow tiles' unrolled steps");
+SmallTile small_plan(int64_t m, int64_t n, int64_t k) {
   SmallTile t;
   if (m <= 4 || k % (128 * kSpU) || m * k >= (int64_t(1) << 31) || n * k >= (int64_t(1) << 31)) return t;
   constexpr int cand[4][2] = {{64, 64}, {80, 32}, {96, 32}, {64, 32}};
@@ -882,19 +888,16 @@ SmallTile small_plan(int64_t m, int64_t n, int64_t k, bool any_count = false) {
       return t;
     }
   }
-  // Short m (no candidate reaches 192 workgroups): the candidate with the
-  // most workgroups, if it has at least 64 (the row-major kernel's 64 x 128
-  // tiles give no more) or there is no row-major weight (any_count).
-  int64_t most = any_count ? 0 : 63;
-  for (const auto& c : cand) {
-    if (n % (4 * c[1]) || c[0] == 80) continue;
-    const int64_t tiles = (m + c[0] - 1) / c[0] * (n / (4 * c[1]));
-    if (tiles > most && tiles <= 512) {
-      most = tiles;
-      t.bm = c[0];
-      t.cw = c[1];
-    }
-  }
+  // Grids of 64 x 128 tiles short of 192 workgroups: 64 x 64 tiles (four weight
+  // and activation register stages) where they make at least 128, else 32 x 64. A
+  // workgroup's time per k step is latency, not products, so more and narrower
+  // workgroups are what fills the GPU; the same bits. Weights streamed, before (64 x
+  // 128) -> after: 320 x 6144 x 2048 (m x k x n) 21.4 -> 14.8 us, 320 x 4096 x 2560
+  // 16.1 -> 10.9, 576 x 6144 x 2048 21.2 -> 20.1, 320 x 2048 x 2048 7.8 -> 5.8; 32 x 64
+  // against 64 x 64: 176 x 6144 x 2048 10.8 against 13.7, 64 x 4096 x 4096 9.6 against
+  // 11.8, and the other way round at 320 x 6144 x 2048, 15.5 against 14.8.
+  if (n % 128 == 0 && (m + 63) / 64 * (n / 128) < 192)
+    return (m + 63) / 64 * (n / 64) >= 128 ? SmallTile{64, 16} : SmallTile{32, 16};
   return t;
 }
 
@@ -903,8 +906,10 @@ void launch_small(const void* qa, const float* sa, int sa_rows, const void* qw_p
                   void* y, int64_t ldy, int64_t m, int64_t n, int64_t k, hipStream_t st) {
   const int64_t tm = (m + BM - 1) / BM, tn = n / (4 * CW);
   // The 80 x 128 tile (the 8B o projection at 576 tokens) on pk_mainloop_pf.
-  constexpr bool pf = BM == 80 && CW == 32;
-  hipLaunchKernelGGL((gemm_fp8_split_packed_kernel<BM, CW, kSpP, kSpD, kSpG, 1, pf>), dim3((unsigned)(tm * tn)),
+  // The narrow tiles too, with four register stages instead of two.
+  constexpr bool narrow = CW == 16, pf = narrow || (BM == 80 && CW == 32);
+  constexpr int P = narrow ? 4 : kSpP, D = narrow ? 4 : kSpD;
+  hipLaunchKernelGGL((gemm_fp8_split_packed_kernel<BM, CW, P, D, kSpG, 1, pf>), dim3((unsigned)(tm * tn)),
                      dim3(kThreads), 0, st, (const uint8_t*)qa, sa, sa_rows, (const uint8_t*)qw_packed, sw, sw_cols,
                      (bf16_t*)y, ldy, (int)m, (int)n, (int)k, (int)tm, (int)tn, (float*)nullptr);
 }
@@ -1538,13 +1543,17 @@ extern "C" int ff_gemm_fp8_pk(const void* qa, const float* sa, int sa_rows, cons
   const SplitPlan plan = pk ? split_plan(m, n, k) : SplitPlan{};
   const int s = plan.s;
   if (s == 0) {
-    const SmallTile t = pk ? small_plan(m, n, k, !qw) : SmallTile{};
+    const SmallTile t = pk ? small_plan(m, n, k) : SmallTile{};
     if (t.bm == 64 && t.cw == 64)
       launch_small<64, 64>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, st);
     else if (t.bm == 80)
       launch_small<80, 32>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, st);
     else if (t.bm == 96)
       launch_small<96, 32>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, st);
+    else if (t.bm == 64 && t.cw == 16)
+      launch_small<64, 16>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, st);
+    else if (t.bm == 32)
+      launch_small<32, 16>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, st);
     else if (t.bm == 64)
       launch_small<64, 32>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, st);
     else if (qw)

@@ -422,6 +422,41 @@ def test_gemm_fp8_pk_matches_rowmajor(gpu, m, n, k, bm, splits):
                          "gemm_fp8_pk split 4")
 
 
+# grids of 64 x 128 tiles short of the GPU: 32 x 64 tiles (5 .. 65 rows, one row tile
+# and its edges; the smallest n and k) and 64 x 64 tiles from 128 of them up (ragged
+# last row tile; an odd number of unrolled k blocks); 176 x 6144 x 4096 runs unsplit
+@pytest.mark.parametrize("m,n,k", [(5, 128, 512), (31, 128, 1536), (32, 2048, 2048), (33, 2048, 512), (65, 1024, 1024),
+                                   (300, 1024, 512), (320, 2048, 6144), (257, 2048, 1536), (576, 2048, 2048),
+                                   (320, 2560, 4096), (176, 6144, 4096)])
+@pytest.mark.parametrize("rows", [True, False])
+def test_gemm_fp8_pk_narrow_tiles(gpu, m, n, k, rows):
+    """The narrow packed tiles: bit for bit ff_gemm_fp8 on the row-major codes, with
+    per-token / per-channel and with scalar scales, with and without the row-major
+    weight given, and no workspace."""
+    from fastforward_amd._lib import call, ptr, stream
+    from fastforward_amd.linear import FP8Linear, gemm_pk_workspace
+    x = (torch.randn(m, k, generator=_g(160)) * 2).to(BF16).to(DEV)
+    op = FP8Linear((torch.randn(n, k, generator=_g(161)) * 0.03).to(BF16).to(DEV), keep_rowmajor=True)
+    qa, sa = op.quantize(x)
+    sw = op.scale
+    if not rows:
+        sa, sw = sa[:1].clone(), sw.reshape(-1)[:1].clone()
+    if m > 256 or (m, n) == (176, 6144):
+        assert gemm_pk_workspace(m, n, k) == 0
+    r = 1 if rows else 0
+    ref = torch.empty(m, n, device=DEV, dtype=BF16)
+    call("ff_gemm_fp8", ptr(qa), ptr(sa), r, ptr(op.weight), ptr(sw), r, ptr(ref), n, m, n, k, stream())
+    ws = torch.empty(max(gemm_pk_workspace(m, n, k), 256), device=DEV, dtype=torch.uint8)
+    for w in (op.weight, None):
+        y = torch.full((m, n), float("nan"), device=DEV, dtype=BF16)
+        call("ff_gemm_fp8_pk", ptr(qa), ptr(sa), r, ptr(w), ptr(op.packed), ptr(sw), r, ptr(y), n, m, n, k, ptr(ws),
+             ws.numel(), stream())
+        if gemm_pk_workspace(m, n, k) == 0:
+            assert torch.equal(y, ref)
+        else:   # short m, k split: only the fp32 order of the partials differs
+            assert int(bf16_ulps(y, ref).max()) <= 1
+
+
 @pytest.mark.parametrize("m,n,k,static,deep", [(576, 4096, 12288, False, True), (576, 4096, 12288, True, False),
                                                (500, 4096, 12288, False, False), (300, 2048, 8192, True, True),
                                                (576, 4096, 4096, False, False), (1, 4096, 12288, False, False),
