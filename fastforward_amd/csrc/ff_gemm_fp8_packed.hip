@@ -770,7 +770,7 @@ constexpr int kSpU = lcm3(kSpP, kSpD, 2 * kSpG);
 
 // The plain packed GEMM's plan for an m x n x k product: row tile bm (x 256
 // weight rows) and k splits s (1: unsplit, 0: the kernel does not take it).
-// One launch when 144-row tiles fill the GPU, else 144-row tiles with k split
+// One launch, of the row tile that wastes least, when 144-row tiles fill the GPU, else 144-row tiles with k split
 // when k is long enough that the extra reduction pays off (the 8B down
 // projection, 576 x 4096 x 12288); shorter k takes small_plan's tiles (below)
 // or the row-major kernels. ff_set_tuning(FF_TUNE_FP8_PK_SPLIT, 100 bm + s)
@@ -807,7 +807,25 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k) {
   if (n % kSpBN) return p;
   const int64_t tiles = (m + kSpBM - 1) / kSpBM * (n / kSpBN);
   if (tiles >= 192) {
-    if (kt % kSpU == 0) p = SplitPlan{kSpBM, 1};
+    // One launch. A round of 256 tiles (one per CU) takes time in proportion to
+    // its rows plus about 16 (prologue, epilogue, barriers), so the row tile is
+    // the one with the fewest rounds x (rows + 16), ties to the 144 rows. Weights
+    // streamed, 144 rows -> chosen: 1024 x 25600 x 5120 (m x n x k) 800 tiles in
+    // four rounds 178 us -> 208 rows, 500 tiles in two, 130 us (176 rows 147, 128
+    // rows 153, 112 rows 160); 1024 x 10240 x 8192 114 -> 73 (176 rows, 240 tiles);
+    // 1024 x 12288 x 4096 65.9 -> 49.6 (208 rows); 1999 x 25600 x 5120 256 -> 234
+    // (208 rows); 2048 x 4096 x 12288 93.0 -> 86.6 and 576 x 12288 x 4096 34.9 ->
+    // 32.0 (128 rows). Every row tile gives the same bits.
+    if (kt % kSpU == 0) {
+      int64_t best = 0;
+      for (const int bm : {kSpBM, 112, 128, 176, 208}) {
+        const int64_t t = (m + bm - 1) / bm * (n / kSpBN), cost = (t + 255) / 256 * (bm + 16);
+        if (p.s == 0 || cost < best) {
+          p = SplitPlan{bm, 1};
+          best = cost;
+        }
+      }
+    }
     return p;
   }
   if (m <= 256) {
@@ -929,7 +947,10 @@ void launch_split(const void* qa, const float* sa, int sa_rows, const void* qw_p
   // 576 tokens) and 64 x 256 tiles split 4, 5 or 6 ways (o and down at 176
   // tokens; 5 and 6 deal their k steps out in pk_mainloop_pf's 2-step blocks).
   constexpr bool pf = (BM == 144 && CW == 64 && S == 4) || (BM == 64 && CW == 64 && S >= 4 && S <= 6);
-  hipLaunchKernelGGL((gemm_fp8_split_packed_kernel<BM, CW, kSpP, kSpD, kSpG, S, pf>),
+  // 208 rows hold 208 accumulator registers a lane: one stage of activation
+  // registers fits beside them, two spill.
+  constexpr int D = BM > 176 ? 1 : kSpD;
+  hipLaunchKernelGGL((gemm_fp8_split_packed_kernel<BM, CW, kSpP, D, kSpG, S, pf>),
                      dim3((unsigned)(tiles_m * tiles_n * S)), dim3(kThreads), 0, st, (const uint8_t*)qa, sa, sa_rows,
                      (const uint8_t*)qw_packed, sw, sw_cols, (bf16_t*)y, ldy, (int)m, (int)n, (int)k, (int)tiles_m,
                      (int)tiles_n, (float*)part);
@@ -950,7 +971,7 @@ void launch_splits(int s, const void* qa, const float* sa, int sa_rows, const vo
   }
 }
 
-// The plan's tile: bm x 4 cw (bm 64 or 144 at cw = kSpCW; 64, 80, 96, 128 or 144 at cw = 32).
+// The plan's tile: bm x 4 cw (bm 64 or 144 at cw = kSpCW, unsplit also 112, 128, 176 or 208; 64, 80, 96, 128 or 144 at cw = 32).
 void launch_plan(const SplitPlan& p, int s, const void* qa, const float* sa, int sa_rows, const void* qw_packed,
                  const float* sw, int sw_cols, void* y, int64_t ldy, int64_t m, int64_t n, int64_t k, void* part,
                  hipStream_t st) {
@@ -965,6 +986,14 @@ void launch_plan(const SplitPlan& p, int s, const void* qa, const float* sa, int
       launch_splits<128, 32>(s, qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, part, st);
     else
       launch_splits<kSpBM, 32>(s, qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, part, st);
+  } else if (p.bm == 112) {
+    launch_split<112, 1>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, part, st);
+  } else if (p.bm == 128) {
+    launch_split<128, 1>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, part, st);
+  } else if (p.bm == 176) {
+    launch_split<176, 1>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, part, st);
+  } else if (p.bm == 208) {
+    launch_split<208, 1>(qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, part, st);
   } else if (p.bm == 64) {
     launch_splits<64>(s, qa, sa, sa_rows, qw_packed, sw, sw_cols, y, ldy, m, n, k, part, st);
   } else {

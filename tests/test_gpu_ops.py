@@ -422,6 +422,28 @@ def test_gemm_fp8_pk_matches_rowmajor(gpu, m, n, k, bm, splits):
                          "gemm_fp8_pk split 4")
 
 
+# unsplit 256-column row tiles, by rounds of 256 workgroups x (rows + 16): 112, 128, 144,
+# 176 and 208 rows, each with whole and ragged last row tiles and the shortest k
+@pytest.mark.parametrize("m,n,k", [(1000, 12800, 512), (1120, 12800, 512), (576, 12288, 512), (640, 12288, 1024),
+                                   (140, 49152, 512), (144, 49152, 1024), (1024, 10240, 1536), (1050, 10240, 512),
+                                   (1024, 25600, 512), (1040, 12288, 1536)])
+def test_gemm_fp8_pk_unsplit_row_tiles(gpu, m, n, k):
+    """The unsplit row tiles: bit for bit ff_gemm_fp8 on the row-major codes, nothing
+    written past the last row, and no workspace."""
+    from fastforward_amd._lib import call, ptr, stream
+    from fastforward_amd.linear import FP8Linear, gemm_pk_workspace
+    x = (torch.randn(m, k, generator=_g(62)) * 2).to(BF16).to(DEV)
+    op = FP8Linear((torch.randn(n, k, generator=_g(63)) * 0.03).to(BF16).to(DEV), keep_rowmajor=True)
+    qa, sa = op.quantize(x)
+    assert gemm_pk_workspace(m, n, k) == 0
+    ref = torch.empty(m, n, device=DEV, dtype=BF16)
+    call("ff_gemm_fp8", ptr(qa), ptr(sa), 1, ptr(op.weight), ptr(op.scale), 1, ptr(ref), n, m, n, k, stream())
+    y = torch.full((m + 1, n), float("nan"), device=DEV, dtype=BF16)
+    call("ff_gemm_fp8_pk", ptr(qa), ptr(sa), 1, ptr(op.weight), ptr(op.packed), ptr(op.scale), 1, ptr(y), n,
+         m, n, k, 0, 0, stream())
+    assert torch.equal(y[:m], ref) and bool(y[m].isnan().all())
+
+
 # grids of 64 x 128 tiles short of the GPU: 32 x 64 tiles (5 .. 65 rows, one row tile
 # and its edges; the smallest n and k) and 64 x 64 tiles from 128 of them up (ragged
 # last row tile; an odd number of unrolled k blocks); 176 x 6144 x 4096 runs unsplit
