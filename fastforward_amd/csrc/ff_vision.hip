@@ -749,39 +749,40 @@ __global__ __launch_bounds__(kThreads) void vision_vt_kernel(const bf16_t* __res
 }
 
 // The rotary of vision_rope_block for the packed qkv output, two 8-column
-// groups (two 16-byte stores) per thread: thread -> (q or k, token, head,
-// group pair c and c + 64 of the 128-column output row, c in 0, 8, .., 56);
-// the partners (hd / 2 away, hd % 8 == 0 so each 4-column half of a group
-// lies on one side of hd / 2) come as two 8-byte loads, cos / sin as two
-// 16-byte loads each; both groups' loads are issued before either's
+// groups (two 16-byte stores) of q and the same two of k per thread: thread ->
+// (token, head, group pair c and c + 64 of the 128-column output row, c in 0,
+// 8, .., 56); the partners (hd / 2 away, hd % 8 == 0 so each 4-column half of a
+// group lies on one side of hd / 2) come as two 8-byte loads, cos / sin as two
+// 16-byte loads each, read once for q and k; all loads are issued before any
 // arithmetic. The same two fp32 products and sum per element, rounded once.
 __device__ __forceinline__ void vision_rope8_block(int64_t blk, const bf16_t* __restrict__ qkv, int64_t ts,
                                                    const float* __restrict__ cos, const float* __restrict__ sin,
                                                    bf16_t* __restrict__ yq, bf16_t* __restrict__ yk, int n,
                                                    int heads, int hd) {
-  const int64_t i = blk * kThreads + threadIdx.x;
-  const int64_t per = (int64_t)n * heads * 8;
-  if (i >= 2 * per) return;
-  const bool isk = i >= per;
-  const int64_t r = isk ? i - per : i;
+  const int64_t r = blk * kThreads + threadIdx.x;
+  if (r >= (int64_t)n * heads * 8) return;
   const int64_t th = r >> 3;
   const int head = (int)(th % heads);
   const int64_t tok = th / heads;
-  bf16_t* row = (isk ? yk : yq) + ((int64_t)head * n + tok) * 128;
-  const bf16_t* xr = qkv + tok * ts + (int64_t)(isk ? heads + head : head) * hd;
+  const int64_t orow = ((int64_t)head * n + tok) * 128;
+  const bf16_t* xq = qkv + tok * ts + (int64_t)head * hd;
+  const int64_t kofs = (int64_t)heads * hd;
   const int half = hd / 2;
-  u32x4 xv[2];
-  u32x2 pv[2][2];
+  u32x4 xv[2][2];
+  u32x2 pv[2][2][2];
   float4 cv[2][2], sv[2][2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int c = (int)(r & 7) * 8 + 64 * u;
     if (c < hd) {
-      xv[u] = *reinterpret_cast<const u32x4*>(xr + c);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) xv[t][u] = *reinterpret_cast<const u32x4*>(xq + t * kofs + c);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int cc = c + 4 * h;
-        pv[u][h] = *reinterpret_cast<const u32x2*>(xr + (cc < half ? cc + half : cc - half));
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          pv[t][u][h] = *reinterpret_cast<const u32x2*>(xq + t * kofs + (cc < half ? cc + half : cc - half));
         cv[u][h] = *reinterpret_cast<const float4*>(cos + tok * hd + cc);
         sv[u][h] = *reinterpret_cast<const float4*>(sin + tok * hd + cc);
       }
@@ -791,42 +792,55 @@ __device__ __forceinline__ void vision_rope8_block(int64_t blk, const bf16_t* __
   for (int u = 0; u < 2; ++u) {
     const int c = (int)(r & 7) * 8 + 64 * u;
     if (c >= hd) {
-      *reinterpret_cast<u32x4*>(row + c) = u32x4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(yq + orow + c) = u32x4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(yk + orow + c) = u32x4{0u, 0u, 0u, 0u};
       continue;
     }
-    float x8[8], p8[8], c8[8], s8[8];
-    unpack8(xv[u], x8);
+    float c8[8], s8[8];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const bool lo = c + 4 * h < half;
-      const float pf[4] = {bf16_to_f32(pv[u][h].x & 0xFFFFu), bf16_to_f32(pv[u][h].x >> 16),
-                           bf16_to_f32(pv[u][h].y & 0xFFFFu), bf16_to_f32(pv[u][h].y >> 16)};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) p8[4 * h + e] = lo ? -pf[e] : pf[e];
       c8[4 * h] = cv[u][h].x; c8[4 * h + 1] = cv[u][h].y; c8[4 * h + 2] = cv[u][h].z; c8[4 * h + 3] = cv[u][h].w;
       s8[4 * h] = sv[u][h].x; s8[4 * h + 1] = sv[u][h].y; s8[4 * h + 2] = sv[u][h].z; s8[4 * h + 3] = sv[u][h].w;
     }
-    float o[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = x8[e] * c8[e] + p8[e] * s8[e];
-    *reinterpret_cast<u32x4*>(row + c) = pack8(o);
+    for (int t = 0; t < 2; ++t) {
+      float x8[8], p8[8], o[8];
+      unpack8(xv[t][u], x8);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bool lo = c + 4 * h < half;
+        const u32x2 pw = pv[t][u][h];
+        const float pf[4] = {bf16_to_f32(pw.x & 0xFFFFu), bf16_to_f32(pw.x >> 16), bf16_to_f32(pw.y & 0xFFFFu),
+                             bf16_to_f32(pw.y >> 16)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p8[4 * h + e] = lo ? -pf[e] : pf[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = x8[e] * c8[e] + p8[e] * s8[e];
+      *reinterpret_cast<u32x4*>((t ? yk : yq) + orow + c) = pack8(o);
+    }
   }
 }
 
 // Both of the above for the packed qkv output (n, 3, heads, hd) in one launch:
-// workgroups [0, nrope) rotate q and k into the zero-padded head-major layout
-// (heads, n, 128), the rest write the padded V^T (heads, 128, t_pad).
+// workgroups [0, nvt) write the padded V^T (heads, 128, t_pad), the rest rotate q
+// and k into the zero-padded head-major layout (heads, n, 128).
+// Bound by latency: 39 MB at 2048 patches, 7.8 us at a copy's rate. The V^T
+// workgroups (two dependent passes through LDS) go first, and one thread rotates
+// q and k, so that the 1536 workgroups of 2048 patches are all resident at once
+// where 2560 were not. In graphs of back-to-back launches 13.7 -> 13.2 us at 2048
+// patches, 5.80 -> 5.64 at 400, 8.64 -> 7.85 at 1024 of 64-wide heads.
 __global__ __launch_bounds__(kThreads) void vision_qkv_kernel(const bf16_t* __restrict__ qkv,
                                                               const float* __restrict__ cos,
                                                               const float* __restrict__ sin, bf16_t* __restrict__ yq,
                                                               bf16_t* __restrict__ yk, bf16_t* __restrict__ vt, int n,
-                                                              int t_pad, int heads, int hd, int nrope) {
+                                                              int t_pad, int heads, int hd, int nvt) {
   __shared__ __align__(16) uint16_t tile[64][kVtPitch];
   const int64_t ts = 3 * (int64_t)heads * hd;
-  if ((int)blockIdx.x < nrope) {
-    vision_rope8_block(blockIdx.x, qkv, ts, cos, sin, yq, yk, n, heads, hd);
+  if ((int)blockIdx.x >= nvt) {
+    vision_rope8_block((int)blockIdx.x - nvt, qkv, ts, cos, sin, yq, yk, n, heads, hd);
   } else {
-    vision_vt_block((int)blockIdx.x - nrope, tile, qkv + 2 * (int64_t)heads * hd, ts, hd, vt, n, t_pad, heads, hd);
+    vision_vt_block((int)blockIdx.x, tile, qkv + 2 * (int64_t)heads * hd, ts, hd, vt, n, t_pad, heads, hd);
   }
 }
 
@@ -1191,12 +1205,12 @@ extern "C" int ff_vision_qkv(const void* qkv, const float* cos, const float* sin
   FF_REQUIRE(ff_aligned(qkv, 16) && ff_aligned(cos, 16) && ff_aligned(sin, 16) && ff_aligned(yq, 16) &&
                  ff_aligned(yk, 16) && ff_aligned(vt, 16),
              "ff_vision_qkv: alignment (16 bytes)");
-  const int64_t rope_threads = 2 * n * heads * (128 / 16);
+  const int64_t rope_threads = n * heads * (128 / 16);
   const int nrope = (int)((rope_threads + kThreads - 1) / kThreads);
   const int nvt = (int)(heads * (t_pad / 64));
   hipLaunchKernelGGL(vision_qkv_kernel, dim3((unsigned)(nrope + nvt)), dim3(kThreads), 0, (hipStream_t)stream,
                      (const bf16_t*)qkv, cos, sin, (bf16_t*)yq, (bf16_t*)yk, (bf16_t*)vt, (int)n, (int)t_pad,
-                     (int)heads, (int)hd, nrope);
+                     (int)heads, (int)hd, nvt);
   FF_LAUNCH_CHECK("ff_vision_qkv");
   return FF_OK;
 }

@@ -414,6 +414,31 @@ def test_vision_qkv_equals_rope_and_vt(gpu):
         assert torch.equal(a, b)
 
 
+# one token, a last rotary workgroup that is partly empty, odd head counts; heads of one
+# 8-column group, of 64 (no group pair past 64), of 72 and of the full 128
+@pytest.mark.parametrize("n,nh,hd", [(1, 1, 8), (5, 3, 64), (63, 3, 72), (64, 2, 120), (130, 16, 128), (400, 16, 72)])
+def test_vision_qkv_sizes(gpu, n, nh, hd):
+    """q, k rotated by two fp32 products and their sum, rounded once; v transposed; zeros past
+    the head width and the tokens. Bit for bit, in torch's fp32 on the CPU."""
+    from fastforward_amd._lib import call, ptr, stream
+    n_pad = (n + 63) // 64 * 64
+    qkv = torch.randn(n, 3, nh, hd, generator=_g(15)).to(BF16)
+    cos, sin = (torch.randn(n, hd, generator=_g(s)) for s in (16, 17))
+    yq, yk = (torch.full((nh, n, 128), float("nan"), device=DEV).to(BF16) for _ in range(2))
+    vt = torch.full((nh, 128, n_pad), float("nan"), device=DEV).to(BF16)
+    qkv_d, cos_d, sin_d = qkv.to(DEV), cos.to(DEV), sin.to(DEV)
+    call("ff_vision_qkv", ptr(qkv_d), ptr(cos_d), ptr(sin_d), ptr(yq), ptr(yk), ptr(vt), n, n_pad, nh, hd, stream())
+    for part, got in ((0, yq), (1, yk)):
+        x = qkv[:, part].float()
+        rot = torch.cat((-x[..., hd // 2:], x[..., :hd // 2]), -1)
+        want = torch.zeros(nh, n, 128, dtype=BF16)
+        want[..., :hd] = (x * cos[:, None] + rot * sin[:, None]).to(BF16).transpose(0, 1)
+        assert torch.equal(got.cpu(), want)
+    want = torch.zeros(nh, 128, n_pad, dtype=BF16)
+    want[:, :hd, :n] = qkv[:, 2].permute(1, 2, 0)
+    assert torch.equal(vt.cpu(), want)
+
+
 def test_vision_vt_layout(gpu):
     from fastforward_amd._lib import call, ptr, stream
     n, nh, hd, n_pad = 100, 4, 72, 128
