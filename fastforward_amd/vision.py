@@ -70,7 +70,8 @@ VISION_PRESETS = {
 class Lin:
     """A bf16 linear: weight (n, k) and bias (n,) on the device, and once
     ``pack`` has run the weight's copy in the packed GEMM's operand order
-    (ff_pack_weight_bf16; ``linear`` then reads it, the same bits)."""
+    (ff_pack_weight_bf16; ``linear`` passes it on, and the k splits of short
+    calls read it)."""
     w: torch.Tensor
     b: torch.Tensor
     p: torch.Tensor = None
