@@ -152,48 +152,6 @@ __device__ __forceinline__ float softmax_block(f32x4 (&s)[4], bool masked, int l
   return alpha;
 }
 
-// The block of the bidirectional attention (the vision tower), which has no
-// schedule to reproduce: the scores' reference m moves only when some query's
-// maximum exceeds its own by more than 2^8 in p (p then stays below 256, and
-// bf16(p), its sum and the products keep their relative precision), so that
-// after the first block alpha is 1 and acc needs no rescale; and (s - m) c2 is
-// one fma. VALU instructions per 16 scores: 64 instead of 114.
-__device__ __forceinline__ float softmax_block_free(f32x4 (&s)[4], bool masked, int lim, float c2, float& m,
-                                                    float& den, u32x4 (&pf)[2]) {
-  if (masked) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (32 * (i >> 1) + 4 * (i & 1) + r > lim) s[i][r] = -INFINITY;
-  }
-  const float mnew = fmaxf(m, max_rows(max16(s)));
-  float alpha = 1.0f;
-  if (__ballot((mnew - m) * c2 > 8.0f)) {  // m = -inf before the first block
-    alpha = __builtin_amdgcn_exp2f((m - mnew) * c2);
-    m = mnew;
-  }
-  const float off = m == -INFINITY ? 0.f : -m * c2;  // every score so far -inf: p = 0
-  float p[16], psum = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], c2, off));
-      p[4 * i + r] = e;
-      psum += e;
-    }
-  den = den * alpha + psum;
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    pf[c].x = pack_bf16x2(p[8 * c + 0], p[8 * c + 1]);
-    pf[c].y = pack_bf16x2(p[8 * c + 2], p[8 * c + 3]);
-    pf[c].z = pack_bf16x2(p[8 * c + 4], p[8 * c + 5]);
-    pf[c].w = pack_bf16x2(p[8 * c + 6], p[8 * c + 7]);
-  }
-  return alpha;
-}
-
 // acc *= alpha (its first DTN 16-column tiles), skipped when no query of the
 // wave changed its max (alpha == 1 exactly leaves acc unchanged).
 template <int DTN = 8>
@@ -766,8 +724,7 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)
       const int tq0 = wq0 + 16 * qt;  // first query of the tile
       const bool masked = CAUSAL ? (kb + 63 > tq0 || kb + 63 >= t) : kb + 63 >= t;
       const int lim = (CAUSAL ? min(tq0 + r16, t - 1) : t - 1) - kb - 8 * g;
-      const float alpha = CAUSAL ? softmax_block(sc[qt], masked, lim, c2, m[qt], den[qt], pf[qt])
-                                 : softmax_block_free(sc[qt], masked, lim, c2, m[qt], den[qt], pf[qt]);
+      const float alpha = softmax_block(sc[qt], masked, lim, c2, m[qt], den[qt], pf[qt]);
       rescale<DTN>(o[qt], alpha);
     }
 #pragma unroll
@@ -982,10 +939,9 @@ extern "C" int ff_attention_full(const void* q, const void* k, const void* vt, v
   // at 1024 patches: 15.0 us; two query tiles a wave 20.1). Past that 4 x 32 queries
   // with the key blocks dealt to two sets of four waves while that is at most one
   // workgroup per CU: every fragment read from LDS feeds two MFMAs, two waves per
-  // SIMD overlap, and a CU stages the keys once (2048 patches: 34.5 us, 4 x 16
-  // queries at two workgroups per CU 36.0; 41.0 before the narrower stages and
-  // softmax_block_free). Else 4 x 32 queries at two workgroups
-  // per CU. ff_set_tuning(FF_TUNE_ATTN_QT, 1 | 2) forces the query tiles per wave.
+  // SIMD overlap, and a CU stages the keys once (2048 patches: 36.0 us, 4 x 16
+  // queries at two workgroups per CU 37.1; 39.8 before the narrower stages). Else
+  // 4 x 32 queries at two workgroups per CU. ff_set_tuning(FF_TUNE_ATTN_QT, 1 | 2) forces the query tiles per wave.
   const int qt_env = ff_tuning(FF_TUNE_ATTN_QT);
   const int64_t w64 = (t + 63) / 64 * heads, w128 = (t + 127) / 128 * heads;
   const int qt = qt_env == 1 || qt_env == 2 ? qt_env : (w64 <= 256 ? 1 : 2);

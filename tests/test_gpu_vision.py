@@ -515,6 +515,69 @@ def test_attention_full_key_split(gpu, n, hd, ramp):
     assert float((got - want).abs().max()) <= (1 / 16 if ramp > 0 else 1 / 64)   # |v| up to 4 with one key dominating
 
 
+def _attention_full(q, k, v):
+    """ff_attention_full of (n, heads, hd) bf16 q, k, v on the host; the output on the host."""
+    from fastforward_amd._lib import call, ptr, stream
+    n, nh, hd = q.shape
+    n_pad = (n + 63) // 64 * 64
+    qd, kd = (torch.zeros(nh, n, 128, dtype=BF16, device=DEV) for _ in range(2))
+    qd[:, :, :hd], kd[:, :, :hd] = q.transpose(0, 1).to(DEV), k.transpose(0, 1).to(DEV)
+    vt = torch.zeros(nh, 128, n_pad, dtype=BF16, device=DEV)
+    vt[:, :hd, :n] = v.permute(1, 2, 0).to(DEV)
+    y = torch.full((n, nh * hd), float("nan"), device=DEV, dtype=BF16)
+    call("ff_attention_full", ptr(qd), ptr(kd), ptr(vt), ptr(y), n, n_pad, nh, hd, float(hd ** -0.5), stream())
+    return y.cpu()
+
+
+# 4 x 16, and past one workgroup per CU, queries of 16 heads; two heads of many patches
+@pytest.mark.parametrize("n,nh,hd", [(130, 3, 72), (1000, 16, 64), (1100, 16, 72), (2300, 2, 128)])
+def test_attention_full_peaked_precision(gpu, n, nh, hd):
+    """Scores of standard deviation 4, where one weight of most queries is near 1: taken
+    against the running maximum, that weight is exactly 1 in bf16. The distance from the
+    64-bit result is then the bf16 rounding of the output and of the lesser weights, which
+    the host computes; 1.1 of it leaves room for the fp32 sums, and a weight that is not
+    1 (any other reference) makes it 1.4 of it."""
+    q, k, v = (torch.randn(n, nh, hd, generator=_g(50 + i)) for i in range(3))
+    q, k, v = (q * 4).to(BF16), k.to(BF16), v.to(BF16)
+    got = _attention_full(q, k, v).double().reshape(n, nh, hd)
+    err = floor = 0.0
+    for h in range(nh):
+        s = q[:, h].double() @ k[:, h].double().T * hd ** -0.5
+        p = torch.exp(s - s.amax(1, keepdim=True))
+        den, vh = p.sum(1, keepdim=True), v[:, h].double()
+        exact = p @ vh / den
+        err += float((got[:, h] - exact).square().sum())
+        floor += float((exact.to(BF16).double() - exact).square().sum())
+        floor += float((p.to(BF16).double() @ vh / den - exact).square().sum())
+    assert err <= 1.1 ** 2 * floor
+
+
+def test_attention_full_rows_stand_alone(gpu):
+    """A query's output is the same bits whatever the other queries of its tile are; and
+    where half of a tile's queries score -inf (a dot product past fp32's range) on the
+    first two key blocks, those get weights of the keys after them and the other half
+    the attention over all keys."""
+    n, nh, hd = 300, 2, 72
+    q, k, v = (torch.randn(n, nh, hd, generator=_g(60 + i)) for i in range(3))
+    q[:, :, 0] = 0
+    k[:128, :, 0] = -3e38
+    q, k, v = (t.to(BF16) for t in (q, k, v))
+    plain = _attention_full(q, k, v)
+    mixed = q.clone()
+    mixed[1::2] *= 5
+    mixed[1::2, :, 0] = 4.0          # 4 x -3e38 is past the fp32 range
+    got = _attention_full(mixed, k, v)
+    assert torch.equal(got[::2], plain[::2])
+    assert bool(torch.isfinite(got.float()).all())
+    k0 = k.clone()
+    k0[:, :, 0] = 0
+    want = OV.attention(q, k0, v, hd ** -0.5).float()
+    assert float((plain.float() - want).norm() / want.norm()) <= 5e-3
+    s = torch.einsum("qhd,khd->hqk", mixed[1::2].double(), k[128:].double()) * hd ** -0.5
+    want = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), v[128:].double()).reshape(-1, nh * hd)
+    assert float((got[1::2].double() - want).norm() / want.norm()) <= 5e-3
+
+
 def test_pos_interp_bit_exact(gpu):
     from fastforward_amd.vision import VisionConfig, interp_taps
     from fastforward_amd._lib import call, ptr, stream
