@@ -543,10 +543,6 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attention_decode_kernel(
 // computed: at 72 dims K dims 64 .. 95 as 4 blocks of 16 rows x 64 B and 80 rows
 // of V^T, 22 KB.
 //
-// KS = 2 (bidirectional only): two sets of NW waves share the queries, set s takes
-// the key blocks s, s + 2, ..; a stage holds one block of each, and the sets'
-// sums are merged through LDS at the end.
-//
 // Grid: one dimension, heaviest query blocks first across all groups; the
 // group is blockIdx % (hq/HPW), so with 8 XCDs taking workgroups round-robin
 // the groups of one kv head stay on one XCD (and its L2).
@@ -556,24 +552,21 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attention_decode_kernel(
 // head dim stored per (query, head) of y, which is (s, hq, DOUT); heads
 // narrower than 128 are zero-padded to 128 in q, k and V^T, which leaves every
 // score and every stored output column exact.
-template <int QT, int HPW, int NS, bool CAUSAL = true, int DOUT = D, bool QOUT = false, int NW = 4, int KS = 1>
-__global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)) void attention_prefill_kernel(
+template <int QT, int HPW, int NS, bool CAUSAL = true, int DOUT = D, bool QOUT = false>
+__global__ __launch_bounds__(kThreads, NS == 2 ? 2 : 1) void attention_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ vt,
     bf16_t* __restrict__ y, int s_len, int t, int t_pad, int hq, int hk, float c2, int nqb, float qinv) {
-  constexpr int QB = 16 * QT * (NW / HPW);
+  constexpr int QB = 16 * QT * (4 / HPW);
   // Head dims past DOUT are zero in q, k and V^T: only the first KST 32-dim
   // steps of q.k and the first DTN 16-dim tiles of P.V are loaded and computed.
   constexpr int KST = (DOUT + 31) / 32, DTN = (DOUT + 15) / 16;
   constexpr int KH = KST == 4 ? 8 : (KST == 3 ? 4 : 0);  // 1 KB blocks of K dims 64 and up
   constexpr int VB = 2 * DTN, BLOCKS = 8 + KH + VB;      // and of V^T, and of a stage
-  constexpr int NT = NW * KS;                            // waves
-  constexpr int PW = (KS * BLOCKS + NT - 1) / NT;        // DMAs per wave and stage
-  constexpr int KB = BLOCKS * 1024, STAGE = KS * KB, VOFF = (8 + KH) * 1024;
+  constexpr int PW = (BLOCKS + 3) / 4;                   // DMAs per wave and stage
+  constexpr int STAGE = BLOCKS * 1024, VOFF = (8 + KH) * 1024;
   static_assert(NS == 2 || NS == 3, "two or three K/V stages");
-  static_assert(KS == 1 || (!CAUSAL && HPW == 1 && !QOUT), "only the bidirectional attention splits keys over waves");
   __shared__ __align__(1024) uint8_t smem[NS * STAGE];
-  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wave = wid % NW, ks = wid / NW;  // query set, share of the key blocks
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
   const int ngroups = hq / HPW;
   const int grp = (int)blockIdx.x % ngroups;
@@ -583,22 +576,21 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)
   const int q0 = qb * QB;
   const int wq0 = q0 + (wave / HPW) * 16 * QT;  // first query of this wave
   const int kend = CAUSAL ? min(t, min(s_len, q0 + QB)) : t;  // keys [0, kend) are visible to some query
-  const int nblocks = (kend + 63) / 64, niter = (nblocks + KS - 1) / KS;
+  const int nblocks = (kend + 63) / 64;
 
-  // Load sources of this lane: the stage's 1 KB blocks id = wid + NT i (past the
+  // Load sources of this lane: the stage's 1 KB blocks b = wave + 4 i (past the
   // last one: the last again, the same bytes to the same place, so that every
-  // wave counts PW loads per stage), id / BLOCKS = which of the stage's KS key
-  // blocks, b = id % BLOCKS: b < 8: K rows [8 b, 8 b + 8), dims 0 .. 63; then dims 64
-  // and up, 8 rows x 128 B (KST 4) or 16 rows x 64 B (KST 3: dims 64 .. 95); then V^T
-  // rows 8 per block. Key blocks past the last one load the last one again.
+  // wave counts PW loads per stage). b < 8: K rows [8 b, 8 b + 8), dims 0 .. 63; then
+  // dims 64 and up, 8 rows x 128 B (KST 4) or 16 rows x 64 B (KST 3: dims 64 .. 95);
+  // then V^T rows 8 per block.
   const bf16_t* kbase = k + (int64_t)kvh * t * D;
   const bf16_t* vbase = vt + (int64_t)kvh * D * t_pad;
-  auto block_of = [&](int i) { return (KS * BLOCKS) % NT ? min(wid + NT * i, KS * BLOCKS - 1) : wid + NT * i; };
+  auto block_of = [&](int i) { return BLOCKS % 4 ? min(wave + 4 * i, BLOCKS - 1) : wave + 4 * i; };
   int k_key[PW], k_col[PW];
   int64_t v_off[PW];
 #pragma unroll
   for (int i = 0; i < PW; ++i) {
-    const int b = block_of(i) % BLOCKS;
+    const int b = block_of(i);
     int key = 8 * (b & 7) + (lane >> 3);
     const int swz = ((key >> 1) & 1) | ((key >> 2) & 6);
     int col = 64 * (b >> 3) + 8 * ((lane & 7) ^ swz);
@@ -612,16 +604,13 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)
     v_off[i] = (int64_t)d * t_pad + 8 * ((lane & 7) ^ ((d >> 1) & 7));
   }
   const uint32_t lds0 = lds_addr(smem);
-  auto issue = [&](int it, int buf) {
+  auto issue = [&](int kb, int buf) {
 #pragma unroll
     for (int i = 0; i < PW; ++i) {
-      const int id = block_of(i);  // wave-uniform
-      const int kb = 64 * (KS == 1 ? it : min(KS * it + id / BLOCKS, nblocks - 1));
-      const uint32_t dst = lds0 + buf * STAGE + (uint32_t)id * 1024;
+      const int b = block_of(i);  // wave-uniform
+      const uint32_t dst = lds0 + buf * STAGE + (uint32_t)b * 1024;
       // K or V^T, known at compile time where round i holds one kind only
-      const bool isk = KS == 1 && NT * (i + 1) <= 8 + KH ? true
-                       : KS == 1 && NT * i >= 8 + KH     ? false
-                                                         : id % BLOCKS < 8 + KH;
+      const bool isk = 4 * (i + 1) <= 8 + KH ? true : 4 * i >= 8 + KH ? false : b < 8 + KH;
       if (isk) lds_dma16(kbase + (int64_t)min(kb + k_key[i], t - 1) * D + k_col[i], dst);
       else lds_dma16(vbase + v_off[i] + kb, dst);
     }
@@ -658,7 +647,7 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)
   // loop would also wait for the prefetches issued there.
 #pragma unroll
   for (int st = 0; st < NS - 1; ++st)
-    if (st < niter) issue(st, st);
+    if (st < nblocks) issue(64 * st, st);
   u32x4 qf[QT][4];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -673,15 +662,14 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)
 #pragma unroll
     for (int st = 0; st < KST; ++st)
       asm volatile("" : : "v"(qf[qt][st].x), "v"(qf[qt][st].y), "v"(qf[qt][st].z), "v"(qf[qt][st].w));
-  for (int it = 0; it < niter; ++it) {
-    if (NS == 3 && it + 1 < niter) wait_vmcnt<PW>();
+  for (int ib = 0; ib < nblocks; ++ib) {
+    if (NS == 3 && ib + 1 < nblocks) wait_vmcnt<PW>();
     else wait_vmcnt<0>();
-    barrier_lds();  // stage it landed for every wave; stage it - 1 fully consumed
-    if (it + NS - 1 < niter) issue(it + NS - 1, (it + NS - 1) % NS);
-    const int kb = 64 * (KS * it + ks);
-    if (KS > 1 && kb >= t) continue;  // wave-uniform: an odd last block is the first share's
+    barrier_lds();  // block ib landed for every wave; block ib - 1 fully consumed
+    if (ib + NS - 1 < nblocks) issue((ib + NS - 1) * 64, (ib + NS - 1) % NS);
+    const int kb = ib * 64;
     if (CAUSAL && (kb >= s_len || kb > wq0 + 16 * QT - 1)) continue;  // wave-uniform: no query of the wave sees it
-    const uint8_t* st_base = smem + (it % NS) * STAGE + ks * KB;
+    const uint8_t* st_base = smem + (ib % NS) * STAGE;
 
     // Every K fragment of the block is read before the first S MFMA, and every
     // V^T fragment right after the last one, so that these LDS reads are in
@@ -735,33 +723,6 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 16 ? 4 : (NS == 2 ? 2 : 1)
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) o[qt][dt] = mfma_bf16(vf[c][dt], pf[qt][c], o[qt][dt]);
       }
-  }
-  // The key shares of one query set are merged through LDS, lane by lane, in the
-  // frame of the larger reference.
-  if constexpr (KS == 2) {
-    static_assert(NW * QT * (DTN + 1) * 1024 <= NS * STAGE, "the shares' sums fit the stages");
-    uint8_t* buf = smem + wave * (QT * (DTN + 1) * 1024) + 16 * lane;
-    barrier_lds();  // every wave is done reading the stages
-    if (ks == 1) {
-#pragma unroll
-      for (int qt = 0; qt < QT; ++qt) {
-#pragma unroll
-        for (int dt = 0; dt < DTN; ++dt) *reinterpret_cast<f32x4*>(buf + (qt * (DTN + 1) + dt) * 1024) = o[qt][dt];
-        *reinterpret_cast<f32x4*>(buf + (qt * (DTN + 1) + DTN) * 1024) = f32x4{m[qt], den[qt], 0.f, 0.f};
-      }
-    }
-    barrier_lds();
-    if (ks == 1) return;
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-      const f32x4 md = *reinterpret_cast<const f32x4*>(buf + (qt * (DTN + 1) + DTN) * 1024);
-      const float mx = fmaxf(m[qt], md[0]);  // share 0 holds key block 0, so it is a score
-      const float a0 = __builtin_amdgcn_exp2f((m[qt] - mx) * c2), a1 = __builtin_amdgcn_exp2f((md[0] - mx) * c2);
-      den[qt] = den[qt] * a0 + md[1] * a1;
-#pragma unroll
-      for (int dt = 0; dt < DTN; ++dt)
-        o[qt][dt] = o[qt][dt] * a0 + *reinterpret_cast<const f32x4*>(buf + (qt * (DTN + 1) + dt) * 1024) * a1;
-    }
   }
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -935,30 +896,25 @@ extern "C" int ff_attention_full(const void* q, const void* k, const void* vt, v
   FF_REQUIRE(ff_aligned(q, 16) && ff_aligned(k, 16) && ff_aligned(vt, 16) && ff_aligned(y, 8),
              "ff_attention_full: alignment");
   const float c2 = (float)((double)scale * 1.4426950408889634);  // scale * log2(e)
-  // 4 waves x 16 queries while that grid is at most one workgroup per CU (16 heads
-  // at 1024 patches: 15.0 us; two query tiles a wave 20.1). Past that 4 x 32 queries
-  // with the key blocks dealt to two sets of four waves while that is at most one
-  // workgroup per CU: every fragment read from LDS feeds two MFMAs, two waves per
-  // SIMD overlap, and a CU stages the keys once (2048 patches: 36.0 us, 4 x 16
-  // queries at two workgroups per CU 37.1; 39.8 before the narrower stages). Else
-  // 4 x 32 queries at two workgroups per CU. ff_set_tuning(FF_TUNE_ATTN_QT, 1 | 2) forces the query tiles per wave.
+  // 4 waves x 16 queries while that grid is at most three workgroups per CU, else 4
+  // waves x 32 queries: half the workgroups, each reading a key block's fragments
+  // once for two tiles. One tile against two, 16 heads of 72 dims: 400 patches 9.3
+  // against 12.5 us, 2048 (two per CU) 39.4 against 39.9, 2304 55.9 against 65.9,
+  // 3072 (three per CU) 79.0 against 86.7, 4096 136 against 117; 64 and 128 dims cross
+  // over at the same grids. Every query sums the key blocks in order, so both give the
+  // same bits. ff_set_tuning(FF_TUNE_ATTN_QT, 1 | 2) forces the tiles per wave.
   const int qt_env = ff_tuning(FF_TUNE_ATTN_QT);
-  const int64_t w64 = (t + 63) / 64 * heads, w128 = (t + 127) / 128 * heads;
-  const int qt = qt_env == 1 || qt_env == 2 ? qt_env : (w64 <= 256 ? 1 : 2);
-  const int ks = qt == 2 && w64 > 256 && w128 <= 256 ? 2 : 1;
-  constexpr int nw = 4;
-  const int qb = 16 * qt * nw;  // one head per workgroup: nw waves x QT tiles of 16 queries
+  const int qt = qt_env == 1 || qt_env == 2 ? qt_env : ((t + 63) / 64 * heads <= 768 ? 1 : 2);
+  const int qb = 16 * qt * 4;  // one head per workgroup: 4 waves x QT tiles of 16 queries
   const int nqb = (int)((t + qb - 1) / qb);
-  const dim3 grid((unsigned)(nqb * heads)), block((unsigned)(64 * nw * ks));
+  const dim3 grid((unsigned)(nqb * heads)), block(kThreads);
   hipStream_t st = (hipStream_t)stream;
-#define FF_FULL(QT, DO, KS)                                                                                   \
-  if (qt == QT && d_out == DO && ks == KS)                                                            \
-    hipLaunchKernelGGL((attention_prefill_kernel<QT, 1, 2, false, DO, false, nw, KS>), grid, block, 0, st,        \
-                       (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)vt, (bf16_t*)y, (int)t, (int)t,         \
-                       (int)t_pad, (int)heads, (int)heads, c2, nqb, 0.f);
-#define FF_FULL_D(QT, KS) FF_FULL(QT, 64, KS) FF_FULL(QT, 72, KS) FF_FULL(QT, 128, KS)
-  FF_FULL_D(1, 1) FF_FULL_D(2, 1) FF_FULL_D(2, 2)
-#undef FF_FULL_D
+#define FF_FULL(QT, DO)                                                                                    \
+  if (qt == QT && d_out == DO)                                                                             \
+    hipLaunchKernelGGL((attention_prefill_kernel<QT, 1, 2, false, DO>), grid, block, 0, st, (const bf16_t*)q, \
+                       (const bf16_t*)k, (const bf16_t*)vt, (bf16_t*)y, (int)t, (int)t, (int)t_pad, (int)heads, \
+                       (int)heads, c2, nqb, 0.f);
+  FF_FULL(1, 64) FF_FULL(2, 64) FF_FULL(1, 72) FF_FULL(2, 72) FF_FULL(1, 128) FF_FULL(2, 128)
 #undef FF_FULL
   FF_LAUNCH_CHECK("ff_attention_full");
   return FF_OK;

@@ -482,16 +482,15 @@ def test_attention_full(gpu, n, nh, hd):
     assert torch.equal(y2, y)
 
 
-# 16 heads: 64 queries a workgroup (1000 tokens, one per CU), and past that the key
-# blocks dealt to two sets of waves: an odd and an even number of 64-key blocks,
-# ragged and full last blocks, each head width
+# 16 heads at one workgroup per CU (1000 tokens) and past that: an odd and an even
+# number of 64-key blocks, ragged and full last blocks, each head width
 @pytest.mark.parametrize("n,hd", [(1000, 72), (1025, 72), (1088, 64), (1100, 128), (1152, 72)])
 @pytest.mark.parametrize("ramp", [0.0, 40.0, float("-inf")])
 def test_attention_full_key_split(gpu, n, hd, ramp):
-    """ff_attention_full against the oracle where its grid splits the keys; with
-    ``ramp`` the scores grow along the keys (by about 4 ramp in natural units), so
-    that the running reference moves many times and the two sets' references
-    differ; with -inf the first two key blocks' scores are -inf (weight 0)."""
+    """ff_attention_full against the oracle over many key blocks; with ``ramp`` the
+    scores grow along the keys (by about 4 ramp in natural units), so that the running
+    maximum moves in every block; with -inf the first two key blocks' scores are -inf
+    (weight 0)."""
     from fastforward_amd._lib import call, ptr, stream
     nh = 16
     q, k, v = (torch.randn(n, nh, hd, generator=_g(50 + i)) for i in range(3))
@@ -550,6 +549,22 @@ def test_attention_full_peaked_precision(gpu, n, nh, hd):
         floor += float((exact.to(BF16).double() - exact).square().sum())
         floor += float((p.to(BF16).double() @ vh / den - exact).square().sum())
     assert err <= 1.1 ** 2 * floor
+
+
+# one, two and more workgroups of 64 queries per CU
+@pytest.mark.parametrize("n,nh,hd", [(400, 16, 72), (1100, 16, 72), (1100, 16, 128), (2300, 16, 64)])
+def test_attention_full_bits_whatever_the_tile(gpu, n, nh, hd):
+    """The key blocks are summed in order for every query, so the built-in choice, one and
+    two query tiles per wave give the same bits at every grid size."""
+    from fastforward_amd._lib import call
+    q, k, v = (torch.randn(n, nh, hd, generator=_g(70 + i)).to(BF16) for i in range(3))
+    ref = _attention_full(q, k, v)
+    for qt in (1, 2):
+        call("ff_set_tuning", 5, qt)  # FF_TUNE_ATTN_QT
+        try:
+            assert torch.equal(_attention_full(q, k, v), ref), qt
+        finally:
+            call("ff_set_tuning", 5, 0)
 
 
 def test_attention_full_rows_stand_alone(gpu):
