@@ -186,6 +186,33 @@ def test_gelu_tanh_every_bf16(gpu):
         assert bool(f(out[0, 0].float()))
 
 
+@pytest.mark.parametrize("tile", [0, 12, 25, 44, 66, "split"])
+def test_gelu_tanh_equals_torch(gpu, tile):
+    """GELU-tanh of every bf16 pattern (as the bias of a zero product): the bits of torch's
+    op on the same device, NaN for NaN and -inf, from the GEMM's epilogue and from the
+    launch that adds a k split's partials."""
+    from fastforward_amd._lib import call
+    from fastforward_amd.vision import Lin, linear, split_workspace
+    vals = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF16).to(DEV)
+    want = torch.nn.functional.gelu(vals, approximate="tanh")
+    if tile == "split":
+        n, k = 8192, 1152
+        assert split_workspace(1, n, k) > 0
+        ws = torch.empty(split_workspace(1, n, k), dtype=torch.uint8, device=DEV)
+    else:
+        n, k, ws = 65536, 64, None
+    w, x = torch.zeros(n, k, dtype=BF16, device=DEV), torch.zeros(1, k, dtype=BF16, device=DEV)
+    if tile != "split":
+        call("ff_set_tuning", FF_TUNE_GEMM_BF16_TILE, tile)
+    try:
+        got = torch.cat([linear(x, Lin(w, b).pack(), act=1, ws=ws)[0] for b in vals.split(n)])
+    finally:
+        call("ff_set_tuning", FF_TUNE_GEMM_BF16_TILE, 0)
+    assert torch.equal(got.isnan(), want.isnan())
+    ok = ~want.isnan()
+    assert torch.equal(got[ok], want[ok])
+
+
 # (m, k, n, act, resid): proj / fc2 of the tower with the residual add in place
 # (64 x 192 tiles), the patch embedding, the mergers' fc1 + GELU (64 x 192) and
 # fc2 (64 x 128), the 128 x 192 and 64 x 256 tiles (GELU-tanh) at row counts
