@@ -1422,7 +1422,7 @@ extern "C" int ff_linear_fp8_rows(const void* x, int64_t x_rs, const float* sa, 
                                   ff_stream_t stream) {
   FF_REQUIRE(x && qw_packed && sw && y, "ff_linear_fp8_rows: null pointer");
   FF_REQUIRE(m >= 1 && m <= 4 && n > 0 && n % 16 == 0 && k >= 512 && k % 128 == 0 && m * k <= FF_LINEAR_FP8_ROWS_MAX &&
-                 n < (int64_t(1) << 31) && x_rs >= k && x_rs % 8 == 0 && ldy >= n,
+                 n * k < (int64_t(1) << 31) && x_rs >= k && x_rs % 8 == 0 && ldy >= n,
              "ff_linear_fp8_rows: bad sizes m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
   FF_REQUIRE(ff_aligned(x, 16) && ff_aligned(qw_packed, 16) && ff_aligned(y, 2), "ff_linear_fp8_rows: alignment");
   hipStream_t s = (hipStream_t)stream;

@@ -228,8 +228,8 @@ int ff_gemm_fp8_pk(const void* qa, const float* sa, int sa_rows, const void* qw,
  * stride x_rs) quantised inside the kernel, per token as ff_quant_rows_fp8 (sa
  * NULL) or as ff_quant_static_fp8 with the multiplier inv and the scale sa[0], then
  * the single-row kernel of ff_gemm_fp8_pk on the packed copy (qw NULL there): the
- * same bits as those two calls. m 1..4, n % 16 == 0, k % 128 == 0, k >= 512, m * k
- * <= FF_LINEAR_FP8_ROWS_MAX (the codes' LDS). Replaces Linear.apply of the
+ * same bits as those two calls. m 1..4, n % 16 == 0, k % 128 == 0, k >= 512, n * k <
+ * 2^31 as there, m * k <= FF_LINEAR_FP8_ROWS_MAX (the codes' LDS). Replaces Linear.apply of the
  * pick-only tail (_family/night_runtime.py:92-105, _legacy/fp8_private.py:33-38). */
 #define FF_LINEAR_FP8_ROWS_MAX 49152
 int ff_linear_fp8_rows(const void* x, int64_t x_rs, const float* sa, float inv, const void* qw_packed,

@@ -72,6 +72,21 @@ def test_tuning_knobs_validate_without_a_gpu(lib_path):
     assert "getenv" not in text
 
 
+def test_linear_fp8_rows_takes_what_the_two_calls_take(lib_path):
+    """Sizes are checked on the host before anything is launched: weights of 2^31 codes
+    and more are refused, as ff_gemm_fp8_pk refuses them without the row-major copy."""
+    from fastforward_amd import _lib
+    _lib.load()
+    buf = (ctypes.c_char * 4096)()
+    p = (ctypes.addressof(buf) + 15) // 16 * 16
+    for m, n, k in ((1, 151936, 16384), (1, 1 << 22, 512), (5, 128, 512), (1, 128, 384), (4, 128, 12288 + 128),
+                    (1, 120, 512), (1, 128, 520)):
+        with pytest.raises(RuntimeError, match="ff_linear_fp8_rows: bad sizes"):
+            _lib.call("ff_linear_fp8_rows", p, k, None, 0.0, p, p, 1, p, n, m, n, k, None)
+    with pytest.raises(RuntimeError, match="ff_gemm_fp8_pk"):
+        _lib.call("ff_gemm_fp8_pk", p, p, 1, None, p, p, 1, p, 151936, 1, 151936, 16384, None, 0, None)
+
+
 def test_w4a16_swiglu_shape_query_without_a_gpu(lib_path):
     """ff_gemm_w4a16_swiglu_fits answers on the host: m > 4 with i % 128 and k % 256,
     or m <= 4 with i % 16 and k % 128; a power-of-two group >= 32 dividing k."""
