@@ -27,6 +27,16 @@ constexpr int kTuneKnobs = 12;
 // Upper bound of each knob's values (index = FF_TUNE_*).
 constexpr int kTuneMax[kTuneKnobs] = {0, 4, 66, 2, 8, 4, 3, 6, 176096, 114408, 8, 114408};
 int g_tuning[kTuneKnobs] = {};
+
+// FF_TUNE_GEMM_BF16_TILE takes the tiles of ff_gemm_bf16 (10 WI + WJ); its three
+// lower values name the tile they named before there were ten.
+int bf16_tile_value(int value) {
+  if (value == 1 || value == 3) return 24;
+  if (value == 2) return 44;
+  for (const int t : {0, 12, 22, 23, 24, 25, 34, 44, 36, 56, 66})
+    if (value == t) return t;
+  return -1;
+}
 }  // namespace
 
 int ff_tuning(int knob) { return knob > 0 && knob < kTuneKnobs ? __atomic_load_n(&g_tuning[knob], __ATOMIC_RELAXED) : 0; }
@@ -34,6 +44,10 @@ int ff_tuning(int knob) { return knob > 0 && knob < kTuneKnobs ? __atomic_load_n
 extern "C" int ff_set_tuning(int knob, int value) {
   FF_REQUIRE(knob > 0 && knob < kTuneKnobs, "ff_set_tuning: unknown knob %d", knob);
   FF_REQUIRE(value >= 0 && value <= kTuneMax[knob], "ff_set_tuning: value %d out of range for knob %d", value, knob);
+  if (knob == FF_TUNE_GEMM_BF16_TILE) {
+    FF_REQUIRE(bf16_tile_value(value) >= 0, "ff_set_tuning: value %d out of range for knob %d", value, knob);
+    value = bf16_tile_value(value);
+  }
   __atomic_store_n(&g_tuning[knob], value, __ATOMIC_RELAXED);
   return FF_OK;
 }

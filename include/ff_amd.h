@@ -40,7 +40,7 @@ int ff_device_check(void);
  * affected entry point is being issued from another thread. */
 #define FF_TUNE_GEMM_FP8_TILE 1   /* ff_gemm_fp8 / _qkv: 1 64x128, 2 128x128, 3 128x128 4-stage, 4 128x256 */
 #define FF_TUNE_GEMM_BF16_TILE 2  /* ff_gemm_bf16: 10 WI + WJ (32 WI x 32 WJ tile): 12, 22, 23, 24, 25, 34, 44, 36,
-                                     56 or 66 (the last two not with a residual) */
+                                     56 or 66 (the last two not with a residual); 1, 2, 3: 24, 44, 24 */
 #define FF_TUNE_W4A16_TILE 3      /* ff_gemm_w4a16*: 1 64x256, 2 192x192 */
 #define FF_TUNE_W4A16_SPLITS 4    /* ff_gemm_w4a16_ws: k splits of the 64x256 tile, 1..8 */
 #define FF_TUNE_ATTN_QT 5         /* ff_attention_vt prefill (1, 2 or 4) / ff_attention_full (1 or 2): query tiles per wave */

@@ -67,6 +67,11 @@ def test_tuning_knobs_validate_without_a_gpu(lib_path):
         _lib.call("ff_set_tuning", 99, 1)
     with pytest.raises(RuntimeError, match="out of range"):
         _lib.call("ff_set_tuning", 4, 9)
+    for tile in (1, 2, 3, 12, 22, 23, 24, 25, 34, 44, 36, 56, 66, 0):   # ff_gemm_bf16's tiles
+        _lib.call("ff_set_tuning", 2, tile)
+    for tile in (4, 11, 13, 33, 55, 65, 67):
+        with pytest.raises(RuntimeError, match="out of range"):
+            _lib.call("ff_set_tuning", 2, tile)
     text = "".join(open(os.path.join(ROOT, "fastforward_amd", "csrc", f)).read()
                    for f in os.listdir(os.path.join(ROOT, "fastforward_amd", "csrc")))
     assert "getenv" not in text
