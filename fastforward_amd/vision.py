@@ -84,19 +84,6 @@ class Lin:
         return self
 
 
-def pack_linears(obj):
-    """``Lin.pack`` on every linear reachable from a weights object (dataclass
-    fields, lists and tuples)."""
-    if isinstance(obj, Lin):
-        obj.pack()
-    elif isinstance(obj, (list, tuple)):
-        for o in obj:
-            pack_linears(o)
-    elif hasattr(obj, "__dataclass_fields__"):
-        for f in obj.__dataclass_fields__:
-            pack_linears(getattr(obj, f))
-
-
 @dataclass
 class Norm:
     w: torch.Tensor
@@ -298,6 +285,18 @@ def split_workspace(m, n, k):
     return b.value
 
 
+def pack_split_linears(w, n, nm):
+    """``Lin.pack`` on the tower's linears whose k is split at ``n`` patches and ``nm``
+    merged tokens: only the k split reads the packed copy (of the 8B tower's 1.1 GB of
+    weights none at 2048 patches)."""
+    calls = [(w.patch, n)]
+    calls += [(lin, n) for b in w.blocks for lin in (b.qkv, b.proj, b.fc1, b.fc2)]
+    calls += [(lin, nm) for mg in (w.merger, *w.deep) for lin in (mg.fc1, mg.fc2)]
+    for lin, m in calls:
+        if split_workspace(m, *lin.w.shape):
+            lin.pack()
+
+
 def layer_norm(x, norm, eps, out=None):
     rows, h = x.shape
     y = torch.empty((rows, h), device=x.device, dtype=BF16) if out is None else out
@@ -357,10 +356,10 @@ class VisionRuntime:
         if gh % cfg.merge or gw % cfg.merge:
             raise ValueError("the patch grid must be a whole number of merge blocks")
         self.cfg, self.w = cfg, weights
-        pack_linears(weights)  # packed weight copies for the packed GEMM (once per weights object)
         self.gh, self.gw = gh, gw
         n = gh * gw
         self.n, self.nm = n, n // cfg.merge ** 2
+        pack_split_linears(weights, n, self.nm)  # once per linear, whatever the geometries sharing it
         self.n_pad = (n + 63) // 64 * 64
         dev = weights.pos_embed.device
         H = cfg.hidden

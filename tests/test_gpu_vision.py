@@ -620,6 +620,28 @@ def test_attention_full_rows_stand_alone(gpu):
     assert float((got[1::2].double() - want).norm() / want.norm()) <= 5e-3
 
 
+def test_tower_packs_only_what_its_splits_read(gpu):
+    """A tower holds packed copies of the linears whose k is split at its patch count and
+    of no others; another geometry on the same weights adds its own."""
+    import dataclasses
+    from fastforward_amd.vision import VISION_PRESETS, VisionRuntime, make_vision
+    cfg = dataclasses.replace(VISION_PRESETS["qwen3vl-8b"], depth=1, deepstack=())
+    w = make_vision(cfg, seed=5)
+    blk = w.blocks[0]
+    names = dict(patch=w.patch, qkv=blk.qkv, proj=blk.proj, fc1=blk.fc1, fc2=blk.fc2, m1=w.merger.fc1, m2=w.merger.fc2)
+    rgb = torch.randint(0, 256, (512, 1024, 3), dtype=torch.uint8, generator=_g(80))
+
+    def run(gh, gw):
+        rt = VisionRuntime(cfg, w, gh, gw)
+        rt.set_image(rgb[:16 * gh, :16 * gw].contiguous())
+        return rt.step()[0].clone()
+    tall = run(32, 64)
+    assert [k for k, lin in names.items() if lin.p is not None] == []
+    run(20, 20)
+    assert [k for k, lin in names.items() if lin.p is not None] == ["patch", "proj", "fc2", "m1", "m2"]
+    assert torch.equal(run(32, 64), tall)
+
+
 def test_pos_interp_bit_exact(gpu):
     from fastforward_amd.vision import VisionConfig, interp_taps
     from fastforward_amd._lib import call, ptr, stream
