@@ -85,6 +85,20 @@ def _assert_within(got, want, slack, what):
     assert eq >= 0.9, f"{what}: only {eq:.3f} of the elements equal the oracle's"
 
 
+def _assert_epilogues(x, w, b, h, run):
+    """The bf16 linear's outputs against references of their own: the plain product within
+    the fp32-accumulation bound of the 64-bit one, and from its bf16 values v, bit for
+    bit, the activations (torch's ops on v) and the residual add (bf16(h + v)).
+    run(act, resid) -> the output; h None: no residual. All on the device."""
+    exact, bound = _linear_bound(x.cpu(), w.cpu(), b.cpu())
+    v = run(0, None)
+    assert bool(((v.cpu().to(torch.float64) - exact).abs() <= bound).all())
+    assert torch.equal(run(1, None), torch.nn.functional.gelu(v, approximate="tanh"))
+    assert torch.equal(run(2, None), torch.nn.functional.gelu(v))
+    if h is not None:
+        assert torch.equal(run(0, h), (h.float() + v.float()).to(BF16))
+
+
 @pytest.mark.parametrize("m,n,k", [(300, 256, 1152), (64, 3456, 1152), (513, 1152, 4352), (2048, 512, 1536)])
 def test_gemm_bf16_plain(gpu, m, n, k):
     from fastforward_amd.vision import Lin, linear
@@ -136,8 +150,8 @@ BF16_TILES = [12, 22, 23, 24, 25, 34, 44, 36, 56, 66]
 @pytest.mark.parametrize("m,n,k", [(1, 4, 64), (33, 100, 128), (191, 196, 384), (193, 320, 448), (385, 1160, 1152)])
 def test_gemm_bf16_every_tile(gpu, m, n, k):
     """ff_gemm_bf16 with each tile forced: bit-equal to the first one (the same
-    products in the same order), which is inside the fp32-accumulation bound; the
-    same for each activation and for a residual added in place."""
+    products in the same order), whose outputs are checked on their own; the same for
+    each activation and for a residual added in place."""
     from fastforward_amd._lib import call
     from fastforward_amd.vision import Lin, linear
     x = torch.randn(m, k, generator=_g(m + 21)).to(BF16)
@@ -155,8 +169,7 @@ def test_gemm_bf16_every_tile(gpu, m, n, k):
         finally:
             call("ff_set_tuning", FF_TUNE_GEMM_BF16_TILE, 0)
     ref = run(BF16_TILES[0])
-    exact, bound = _linear_bound(x, w, b)
-    assert bool(((ref[0].cpu().to(torch.float64) - exact).abs() <= bound).all())
+    _assert_epilogues(x, w, b, h, lambda act, resid: ref[3] if resid is not None else ref[act])
     for tile in BF16_TILES[1:] + [0]:
         for a, c in zip(run(tile), ref):
             assert torch.equal(a, c), tile
@@ -213,12 +226,10 @@ def test_gelu_tanh_equals_torch(gpu, tile):
     assert torch.equal(got[ok], want[ok])
 
 
-# (m, k, n, act, resid): proj / fc2 of the tower with the residual add in place
-# (64 x 192 tiles), the patch embedding, the mergers' fc1 + GELU (64 x 192) and
-# fc2 (64 x 128), the 128 x 192 and 64 x 256 tiles (GELU-tanh) at row counts
-# whose grids they fill, ragged row counts and an odd number of 128-k steps
-# (k 1152); the tower's qkv and fc1 (grids past one round), n = 1000 and 1000
-# rows fall back to the LDS-staged kernel.
+# (m, k, n, act, resid): proj / fc2 of the tower with the residual add in place, the
+# patch embedding, the mergers' fc1 + GELU and fc2, row and column counts of the 2B
+# tower, ragged row counts, an odd number of 128-k steps (k 1152), the tower's qkv and
+# fc1 (GELU-tanh), and n = 1000, which no tile divides
 PK_VISION = [(2048, 1152, 1152, 0, True), (2048, 4352, 1152, 0, True), (2048, 1536, 1152, 0, False),
              (512, 4608, 4608, 2, False), (512, 4608, 4096, 0, False), (1536, 1152, 3456, 0, False),
              (1024, 1152, 4096, 1, False), (2000, 4352, 1152, 0, True), (2048, 1152, 3456, 0, False),
@@ -227,36 +238,36 @@ PK_VISION = [(2048, 1152, 1152, 0, True), (2048, 4352, 1152, 0, True), (2048, 15
 
 @pytest.mark.parametrize("m,k,n,act,resid", PK_VISION)
 def test_gemm_bf16_packed_equals_rowmajor(gpu, m, k, n, act, resid):
-    """linear() on a packed Lin (ff_gemm_bf16_pk: weights from the operand-order
-    copy straight into the MFMA operands) == the LDS-staged kernel on the
-    row-major weight, bit for bit, with every epilogue (bias, GELU-tanh,
-    GELU-erf, residual add in place)."""
+    """linear() at the tower's sizes with every epilogue (bias, GELU-tanh, GELU-erf,
+    residual add in place), on a Lin that holds a packed copy and one that does not: the
+    unsplit product reads the row-major weight either way and gives the outputs of
+    ``_assert_epilogues``."""
     from fastforward_amd.vision import Lin, linear
     x = torch.randn(m, k, generator=_g(m + n)).to(BF16).to(DEV)
     w = (torch.randn(n, k, generator=_g(k)) * 0.03).to(BF16).to(DEV)
     b = (torch.randn(n, generator=_g(n + 2)) * 0.1).to(BF16).to(DEV)
     h = torch.randn(m, n, generator=_g(n + 3)).to(BF16).to(DEV) if resid else None
-    outs = []
-    for lin in (Lin(w, b), Lin(w, b).pack()):
-        if resid:
-            y = h.clone()
-            linear(x, lin, act=act, resid=y, out=y)
-        else:
-            y = linear(x, lin, act=act)
-        outs.append(y)
-    assert (outs[1] is not None) and not torch.isnan(outs[1].float()).any()
-    assert torch.equal(outs[0], outs[1])
+
+    def run(a, r):
+        outs = []
+        for lin in (Lin(w, b), Lin(w, b).pack()):
+            y = None if r is None else r.clone()
+            outs.append(linear(x, lin, act=a, resid=y, out=y))
+        assert torch.equal(outs[0], outs[1])
+        return outs[0]
+    _assert_epilogues(x, w, b, h, run)
+    assert not torch.isnan(run(act, h).float()).any()
 
 
 @pytest.mark.parametrize("m,k,n", [(2048, 1152, 1152), (2000, 1536, 1152)])
 @pytest.mark.parametrize("pad", [8, 4])
 def test_gemm_bf16_packed_strided_residual(gpu, m, k, n, pad):
-    """The packed kernel's residual add with the residual a strided view
-    (row stride n + pad elements) and the output a separate array: pad 8 keeps
-    the residual rows 16-byte aligned (the epilogue reads the tile that was
-    copied into LDS ahead of the main loop), pad 4 does not (it reads global
-    memory); both == the LDS-staged kernel on the row-major weight, bit for bit,
-    and the residual is left unchanged."""
+    """The residual add with the residual a strided view (row stride n + pad elements) and
+    the output a separate array, on every tile that takes a residual: pad 8 keeps the
+    residual rows 16-byte aligned (the epilogue reads the tile that was copied into LDS
+    during the main loop), pad 4 does not (it reads global memory); both are bf16(h + v)
+    of the product v without a residual, bit for bit, and the residual is unchanged."""
+    from fastforward_amd._lib import call
     from fastforward_amd.vision import Lin, linear
     x = torch.randn(m, k, generator=_g(m + n + 11)).to(BF16).to(DEV)
     w = (torch.randn(n, k, generator=_g(k + 12)) * 0.03).to(BF16).to(DEV)
@@ -265,9 +276,14 @@ def test_gemm_bf16_packed_strided_residual(gpu, m, k, n, pad):
     h = wide[:, pad: pad + n]
     assert h.stride(0) == n + pad and (h.data_ptr() % 16 == 0 and h.stride(0) % 8 == 0) == (pad == 8)
     before = wide.clone()
-    outs = [linear(x, lin, resid=h) for lin in (Lin(w, b), Lin(w, b).pack())]
-    assert not torch.isnan(outs[1].float()).any()
-    assert torch.equal(outs[0], outs[1])
+    want = (h.float() + linear(x, Lin(w, b)).float()).to(BF16)
+    for tile in [0] + BF16_TILES[:8]:
+        call("ff_set_tuning", FF_TUNE_GEMM_BF16_TILE, tile)
+        try:
+            outs = [linear(x, lin, resid=h) for lin in (Lin(w, b), Lin(w, b).pack())]
+        finally:
+            call("ff_set_tuning", FF_TUNE_GEMM_BF16_TILE, 0)
+        assert torch.equal(outs[0], want) and torch.equal(outs[1], want), tile
     assert torch.equal(wide, before)
 
 
