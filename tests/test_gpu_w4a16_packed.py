@@ -10,6 +10,8 @@ differs (|difference| <= 1 bf16 ulp + 2^-21 sum |x w|, under 1% of outputs
 differing). Every shape is also held to the fp64 product
 with the exactly dequantised weight (relative RMS <= 5e-3, worst element <=
 0.05 of the output RMS), as the LDS-staged kernel's tests are."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -53,14 +55,25 @@ def _unsplit_lds(op, x, tuning):
         tuning(FF_TUNE_W4A16_SPLITS, 0)
 
 
-def _pk_splits(m, n, k):
-    """Splits the packed plan takes (mirrors w4pk_plan for the tested shapes)."""
-    tm = (m + 143) // 144
-    if n % 384 == 0 and tm * (n // 384) >= 192:
-        return 1
-    tiles = tm * (n // 256)
-    s = 1 if tiles >= 192 else 256 // tiles
-    return max(1, min(s, 8, k // 256))
+def _pk_plan(m, n, k, forced=0):
+    """(row-tile height, splits) of the packed plain product (mirrors w4pk_plan for
+    the tested shapes; forced: FF_TUNE_W4A16_SPLITS)."""
+    if n % 384 == 0 and -(-m // 144) * (n // 384) >= 192:
+        return 144, 1
+    pairs, plans = k // 256, []
+    for bm in (144, 128, 112, 96):
+        tiles = -(-m // bm) * (n // 256)
+        s = max(1, min(forced or (1 if tiles >= 192 else 256 // tiles), 8, pairs))
+        plans.append((-(-tiles * s // 256) * -(-pairs // s) * (bm + 16), bm, s))
+    _, bm, s = min(plans, key=lambda p: p[0])    # the first, tallest, of equals
+    return bm, s
+
+
+def _swiglu_rows(m, i):
+    """Row-tile height of the packed SwiGLU product (mirrors w4_swiglu_bm)."""
+    cw = 96 if i % 192 == 0 else 64
+    return min((144, 128, 112, 96) + ((160,) if cw == 96 else ()),
+               key=lambda bm: -(-(-(-m // bm) * (i // (2 * cw))) // 256) * (bm + 16))
 
 
 def test_pack_weight_int4_layout(gpu):
@@ -101,7 +114,7 @@ def test_w4a16_packed_vs_lds_kernel_and_exact(gpu, tuning, m, k, n, sym, group):
     assert all(torch.equal(outs[0], o) for o in outs[1:])
     dq = O.int4_dequant(op.packed.cpu(), op.scales.cpu(), group).double()
     ref = _unsplit_lds(op, xd, tuning)
-    if m > 4 and _pk_splits(m, n, k) == 1:
+    if m > 4 and _pk_plan(m, n, k)[1] == 1:
         assert torch.equal(outs[0], ref), (m, k, n)
     else:
         # adding the splits' partials reassociates the fp32 sum: an absolute
@@ -119,16 +132,17 @@ def test_w4a16_packed_vs_lds_kernel_and_exact(gpu, tuning, m, k, n, sym, group):
     assert float((y - exact).abs().max() / rms) <= 0.05
 
 
-# row tiles of 96, 112, 128 and 144 rows: full, one row short, one row past
+# short grids, where the 96-row tiles cost least whatever m: full, ragged and many tiles
 @pytest.mark.parametrize("m", [5, 96, 97, 111, 112, 127, 128, 129, 143, 176, 192, 200, 224, 255, 289])
 @pytest.mark.parametrize("sym,group", [(True, 128), (False, 32)])
 def test_w4a16_packed_row_tiles(gpu, tuning, m, sym, group):
-    """Every row-tile height of the packed kernels at its edges: the plain product
-    with k unsplit equals the LDS-staged kernel bit for bit, the SwiGLU form the
-    unfused op sequence on it, the split product the exact one (as above)."""
+    """The 96-row tile of the packed kernels: the plain product with k unsplit equals
+    the LDS-staged kernel bit for bit, the SwiGLU form the unfused op sequence on it,
+    the split product the exact one (as above)."""
     from fastforward_amd import ops
     from fastforward_amd.linear import Int4
     k, n = 1024, 512
+    assert _pk_plan(m, n, k)[0] == _pk_plan(m, n, k, 1)[0] == _swiglu_rows(m, n // 2) == 96
     x = torch.randn(m, k, generator=_g(170)).to(BF16)
     w = (torch.randn(n, k, generator=_g(171)) * 0.02).to(BF16)
     op = Int4(w.to(DEV), group=group, symmetric=sym).pack()
@@ -141,6 +155,63 @@ def test_w4a16_packed_row_tiles(gpu, tuning, m, sym, group):
     tuning(FF_TUNE_W4A16_SPLITS, 0)
     exact = x.double() @ O.int4_dequant(op.packed.cpu(), op.scales.cpu(), group).double().T
     assert float((op(xd).cpu().double() - exact).norm() / exact.norm()) <= 5e-3
+
+
+# (m, n, row tile): grids in which each height makes one round of 256 workgroups and the
+# lower ones two: its last tile of one row (17 for 144 at n 8192, whose 1 is the 16th
+# tile's at n 4096), one row short of full, and full
+HEIGHTS = [(673, 8192, 96), (767, 8192, 96), (768, 8192, 96), (785, 8192, 112), (895, 8192, 112), (896, 8192, 112),
+           (897, 8192, 128), (1023, 8192, 128), (1024, 8192, 128), (1025, 8192, 144), (1151, 8192, 144),
+           (1152, 8192, 144), (2161, 4096, 144)]
+
+
+@pytest.mark.parametrize("m,n,bm", HEIGHTS)
+@pytest.mark.parametrize("sym,group", [(True, 128), (False, 32)])
+def test_w4a16_packed_every_row_tile(gpu, tuning, m, n, bm, sym, group):
+    """Every row-tile height of the packed kernels at its edges: the plain product
+    unsplit equals the LDS-staged kernel bit for bit, split in two it is the exact one
+    within a bf16 rounding, and the SwiGLU form (64-channel wave tiles) equals the unfused
+    op sequence bit for bit."""
+    from fastforward_amd import ops
+    from fastforward_amd._lib import call
+    from fastforward_amd.linear import Int4
+    k = 512
+    x = torch.randn(m, k, generator=_g(172)).to(BF16)
+    w = (torch.randn(n, k, generator=_g(173)) * 0.02).to(BF16)
+    op = Int4(w.to(DEV), group=group, symmetric=sym).pack()
+    xd = x.to(DEV)
+    ref = _unsplit_lds(op, xd, tuning)
+    assert _pk_plan(m, n, k) == (bm, 1) and torch.equal(op(xd), ref)
+    assert (n // 2) % 192 and _swiglu_rows(m, n // 2) == bm
+    assert torch.equal(op.swiglu(xd), ops.swiglu(*ref.chunk(2, -1)))
+    tuning(FF_TUNE_W4A16_SPLITS, 2)
+    need = ctypes.c_int64(0)
+    call("ff_gemm_w4a16_pk_workspace", m, n, k, group, ctypes.byref(need))
+    assert need.value == -(-m // bm) * bm * n * 2 * 4    # two partials of whole tiles
+    y = op(xd).cpu().double()
+    dq = O.int4_dequant(op.packed.cpu(), op.scales.cpu(), group).double()
+    exact = x.double() @ dq.T
+    # each product of bf16 values is exact: the weight's rounding to bf16 and the output's, 2^-9
+    # each, and the fp32 sum
+    bound = 2.0 ** -8 * exact.abs() + (2.0 ** -9 + 2.0 ** -16) * (x.double().abs() @ dq.abs().T)
+    assert bool(((y - exact).abs() <= bound).all())
+    assert float((y - exact).norm() / exact.norm()) <= 5e-3
+
+
+# 96-channel wave tiles: one last row, and full
+@pytest.mark.parametrize("m,bm", [(673, 96), (768, 96), (785, 112), (896, 112), (897, 128), (1024, 128), (1025, 144),
+                                  (1152, 144), (1153, 160), (1280, 160)])
+@pytest.mark.parametrize("sym,group", [(True, 128), (False, 32)])
+def test_w4a16_swiglu_every_row_tile(gpu, tuning, m, bm, sym, group):
+    """The SwiGLU form on 96-channel wave tiles of every height: the unfused op sequence
+    on the LDS-staged kernel, bit for bit."""
+    from fastforward_amd import ops
+    from fastforward_amd.linear import Int4
+    k, i = 512, 6144
+    assert _swiglu_rows(m, i) == bm
+    x = torch.randn(m, k, generator=_g(174)).to(BF16).to(DEV)
+    op = Int4((torch.randn(2 * i, k, generator=_g(175)) * 0.02).to(BF16).to(DEV), group=group, symmetric=sym).pack()
+    assert torch.equal(op.swiglu(x), ops.swiglu(*_unsplit_lds(op, x, tuning).chunk(2, -1)))
 
 
 @pytest.mark.parametrize("n,k", [(256, 256), (256, 512)])
@@ -190,12 +261,12 @@ def test_w4a16_swiglu_gemv_vs_exact(gpu, m, k, i, sym, group):
     assert bool(((unf - want).abs() <= bound).all())
 
 
-# 576 tokens: 144-row tiles; 640: 160-row tiles (one round of 256 workgroups)
+# 576 tokens: 144-row tiles; 640: 160-row tiles (one round of 256 workgroups); the short ones 96-row
 @pytest.mark.parametrize("m,k,i", [(576, 4096, 12288), (640, 4096, 12288), (320, 2048, 6144), (100, 1024, 640)])
 @pytest.mark.parametrize("sym,group", [(True, 128), (False, 32)])
 def test_w4a16_swiglu_packed_equals_unfused(gpu, tuning, m, k, i, sym, group):
     """ff_gemm_w4a16_swiglu_pk == ops.swiglu of the unsplit gate/up product, bit
-    for bit (144 x 384 and 144 x 256 tiles; ragged m)."""
+    for bit (384- and 256-column tiles; ragged m)."""
     from fastforward_amd import ops
     from fastforward_amd.linear import Int4
     x = torch.randn(m, k, generator=_g(73)).to(BF16).to(DEV)
@@ -208,7 +279,10 @@ def test_w4a16_swiglu_packed_equals_unfused(gpu, tuning, m, k, i, sym, group):
     assert torch.equal(h, op.swiglu(x))
 
 
-@pytest.mark.parametrize("m,k,hq,hk", [(576, 4096, 32, 8), (320, 2048, 16, 8), (144, 1024, 8, 4), (100, 1024, 8, 2)])
+# (m, 512, 48, 8): row tiles of 96, 112, 128 and 144 rows, each with one row in its last
+# tile (17 for 144)
+@pytest.mark.parametrize("m,k,hq,hk", [(576, 4096, 32, 8), (320, 2048, 16, 8), (144, 1024, 8, 4), (100, 1024, 8, 2),
+                                       (673, 512, 48, 8), (785, 512, 48, 8), (897, 512, 48, 8), (1025, 512, 48, 8)])
 @pytest.mark.parametrize("sym,group", [(True, 128), (False, 32)])
 def test_w4a16_qkv_fused_equals_unfused(gpu, m, k, hq, hk, sym, group):
     """Int4.qkv (ff_gemm_w4a16_qkv) == the packed QKV GEMM, qk_pair and the V
@@ -219,6 +293,8 @@ def test_w4a16_qkv_fused_equals_unfused(gpu, m, k, hq, hk, sym, group):
     from fastforward_amd.linear import Int4
     d = 128
     n = (hq + 2 * hk) * d
+    if k == 512:
+        assert _pk_plan(m, n, k) == ({673: 96, 785: 112, 897: 128, 1025: 144}[m], 1)
     x = torch.randn(1, m, k, generator=_g(75)).to(BF16).to(DEV)
     w = (torch.randn(n, k, generator=_g(76)) * 0.02).to(BF16)
     op = Int4(w.to(DEV), group=group, symmetric=sym).pack()
