@@ -162,10 +162,13 @@ __device__ __forceinline__ void rescale(f32x4 (&o)[8], float alpha) {
   }
 }
 
-// x / d correctly rounded from r = 1 / d correctly rounded, with the special cases
-// of the IEEE division (v_div_fixup_f32): a row divides all its values by one
-// denominator, so the reciprocal is taken once (4 instructions per value
-// instead of 12).
+// x / d from r = 1 / d correctly rounded (Markstein's correction of a reciprocal
+// product: y = x r, then y + (x - y d) r), with the special cases of the IEEE
+// division (v_div_fixup_f32): a row divides all its values by one denominator, so
+// the reciprocal is taken once (4 instructions per value instead of 12). Correctly
+// rounded while x - y d is exact, for |x| >= 2^-100 and a normal quotient; below that
+// it is a subnormal, and about 4 in 1000 quotients differ from the division in the
+// last fp32 bit, 2^-16 of the bf16 step the output is rounded to.
 __device__ __forceinline__ float div_den(float x, float d, float r) {
   const float y = x * r;
   const float e = __builtin_fmaf(-y, d, x);

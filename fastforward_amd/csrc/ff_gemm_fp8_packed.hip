@@ -770,10 +770,10 @@ constexpr int kSpU = lcm3(kSpP, kSpD, 2 * kSpG);
 
 // The plain packed GEMM's plan for an m x n x k product: row tile bm (x 256
 // weight rows) and k splits s (1: unsplit, 0: the kernel does not take it).
-// One launch, of the row tile that wastes least, when 144-row tiles fill the GPU, else 144-row tiles with k split
-// when k is long enough that the extra reduction pays off (the 8B down
-// projection, 576 x 4096 x 12288); shorter k takes small_plan's tiles (below)
-// or the row-major kernels. ff_set_tuning(FF_TUNE_FP8_PK_SPLIT, 100 bm + s)
+// One launch, of the row tile that wastes least, when 144-row tiles fill the GPU,
+// else 144-row tiles with k split when k is long enough that the extra reduction
+// pays off (the 8B down projection, 576 x 12288 x 4096 as m x k x n); shorter k takes
+// small_plan's tiles (below) or the row-major kernels. ff_set_tuning(FF_TUNE_FP8_PK_SPLIT, 100 bm + s)
 // forces bm in {64, 144} and s in {1, ..., 6, 8} for measurement sweeps.
 // (80-row tiles at two workgroups per CU with half the k splits, fewer fp32
 // partials on the same grid, measured slower: the 8B FP8 step 6.35 -> 6.85 ms
@@ -810,7 +810,7 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k) {
     // One launch. A round of 256 tiles (one per CU) takes time in proportion to
     // its rows plus about 16 (prologue, epilogue, barriers), so the row tile is
     // the one with the fewest rounds x (rows + 16), ties to the 144 rows. Weights
-    // streamed, 144 rows -> chosen: 1024 x 25600 x 5120 (m x n x k) 800 tiles in
+    // streamed, 144 rows -> chosen (m x n x k): 1024 x 25600 x 5120 800 tiles in
     // four rounds 178 us -> 208 rows, 500 tiles in two, 130 us (176 rows 147, 128
     // rows 153, 112 rows 160); 1024 x 10240 x 8192 114 -> 73 (176 rows, 240 tiles);
     // 1024 x 12288 x 4096 65.9 -> 49.6 (208 rows); 1999 x 25600 x 5120 256 -> 234
@@ -837,8 +837,13 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k) {
     // 48 tiles x 5 splits, 240 workgroups (4 splits, 192 workgroups, took the
     // 4.47 ms step to 4.31 ms against small_plan's 64 x 128 tiles for o and
     // 144 x 256 tiles split 8 ways for down). Wider products, which only 2 splits
-    // would fit, run unsplit on small_plan's tiles: 176 x 4096 x 6144 with its
-    // reduction 20.4 us split 2 ways, 18.0 unsplit.
+    // would fit, take the plans below: from k = 8192 144 x 256 tiles split 2, 3, 4 or
+    // 8 ways (or unsplit small tiles at k = 8192), under that small_plan's unsplit
+    // tiles. With their reductions, weights streamed, 64 x 256 tiles split 2 ways ->
+    // those (m x k x n): 193 x 25600 x 5120 68.5 -> 50.6 us, 256 74.1 -> 54.5, 176 72.8
+    // -> 51; 193 x 8192 x 5120 28.0 -> 25.2, 256 30.2 -> 26.7; 256 x 8192 x 7168 31.9
+    // -> 27.2; 224 x 8192 x 8192 31.5 -> 31.3; 176 x 4096 x 6144 20.6 -> 18.0, 256 20.8
+    // -> 15.9; 176 x 5120 x 10240 24.9 -> 19.5; 176 x 8192 x 10240 34 -> 28.4.
     const int64_t t64 = (m + 63) / 64 * (n / kSpBN);
     for (const int sp : {8, 6, 5, 4}) {
       const bool even = sp == 8 || sp == 4;
@@ -971,7 +976,8 @@ void launch_splits(int s, const void* qa, const float* sa, int sa_rows, const vo
   }
 }
 
-// The plan's tile: bm x 4 cw (bm 64 or 144 at cw = kSpCW, unsplit also 112, 128, 176 or 208; 64, 80, 96, 128 or 144 at cw = 32).
+// The plan's tile: bm x 4 cw (bm 64 or 144 at cw = kSpCW, unsplit also 112, 128, 176 or
+// 208; 64, 80, 96, 128 or 144 at cw = 32).
 void launch_plan(const SplitPlan& p, int s, const void* qa, const float* sa, int sa_rows, const void* qw_packed,
                  const float* sw, int sw_cols, void* y, int64_t ldy, int64_t m, int64_t n, int64_t k, void* part,
                  hipStream_t st) {

@@ -207,10 +207,12 @@ int ff_gemm_fp8_swiglu_pk(const void* qa, const float* sa, const void* qw, const
 /* ff_gemm_fp8 with an optional packed copy of the weight (ff_pack_weight_fp8 of
  * qw) and a workspace (no reference counterpart: the down projection of the
  * step, Linear.apply of scaled_qwen_runtime.py:35-39). When qw_packed is given
- * and the shape suits it the weights are read from the packed copy: 144 x 256
- * tiles when 192 or more fill the GPU; with fewer tiles and k >= 8192 k split
+ * and the shape suits it the weights are read from the packed copy: where 192 or
+ * more 144 x 256 tiles fill the GPU, unsplit tiles of 112, 128, 144, 176 or 208 x
+ * 256 (the same bits); with fewer tiles and k >= 8192 144 x 256 tiles with k split
  * 2, 3, 4 or 8 ways; up to 256 tokens 64 x 256 tiles with k split 4, 5, 6 or 8
- * ways; else smaller unsplit tiles (n % 128 == 0, k % 512 == 0). Each split
+ * ways where they fit one round; else smaller unsplit tiles, down to 32 x 64 (n %
+ * 128 == 0, k % 512 == 0). Each split
  * writes its fp32 partial tile to the workspace and a second launch adds the
  * partials in split order (same math as ff_gemm_fp8 up to the fp32 order of
  * adding the partials; repeatable bit for bit). Otherwise this is ff_gemm_fp8
