@@ -843,7 +843,9 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k) {
     // those (m x k x n): 193 x 25600 x 5120 68.5 -> 50.6 us, 256 74.1 -> 54.5, 176 72.8
     // -> 51; 193 x 8192 x 5120 28.0 -> 25.2, 256 30.2 -> 26.7; 256 x 8192 x 7168 31.9
     // -> 27.2; 224 x 8192 x 8192 31.5 -> 31.3; 176 x 4096 x 6144 20.6 -> 18.0, 256 20.8
-    // -> 15.9; 176 x 5120 x 10240 24.9 -> 19.5; 176 x 8192 x 10240 34 -> 28.4.
+    // -> 15.9; 176 x 5120 x 10240 24.9 -> 19.5; 176 x 8192 x 10240 34 -> 28.4. Where
+    // the add_rms launch adds the partials: 193 x 25600 x 5120 71.3 -> 54.5, 193 x 8192 x
+    // 5120 30.7 -> 28.4.
     const int64_t t64 = (m + 63) / 64 * (n / kSpBN);
     for (const int sp : {8, 6, 5, 4}) {
       const bool even = sp == 8 || sp == 4;
