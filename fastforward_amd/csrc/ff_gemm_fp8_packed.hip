@@ -609,10 +609,16 @@ __global__ __launch_bounds__(kThreads, BM <= 96 && !PF ? 2 : 1) void gemm_fp8_sp
   int logical = b;
   if (nblk % kXcds == 0) logical = (b % kXcds) * (nblk / kXcds) + b / kXcds;
   const int tm = logical % tiles_m, rest = logical / tiles_m;  // M fastest: L2 shares weights
-  // Splits outermost: an XCD then reads one split's k range of the activations
-  // instead of all of them (8B down, 576 tokens, with its reduction, weights
-  // streamed: 41.1 -> 40.1 us; 32B 1024 x 25600 x 5120, unsplit, unchanged).
-  const int tn = rest % tiles_n, split = rest / tiles_n;
+  // Splits outermost on tall tiles: an XCD then reads one split's k range of the
+  // activations instead of all of them (with their reductions, weights streamed,
+  // innermost -> outermost, m x k x n: 576 x 12288 x 4096 40.6 -> 39.7 us, 850 83.7 ->
+  // 76.2, 576 x 9728 x 2560 30.8 -> 29.7). Innermost on 64-row tiles (short m, little
+  // activation to read), whose launches are mostly slower the other way round: 100 x
+  // 4096 x 4096 14.3 us against 16.9, 176 16.2 against 16.9, 176 x 4096 x 2560 15.3
+  // against 16.1, 176 x 9728 x 2560 21.8 against 22.5; 176 x 2048 x 4096 14.6 against
+  // 13.4 is the exception.
+  constexpr bool outer = BM >= 96;
+  const int tn = outer ? rest % tiles_n : rest / S, split = outer ? rest / tiles_n : rest % S;
   const int m0 = tm * BM, n0 = tn * BN;
   const int tid = threadIdx.x, wave = tid >> 6;
   // this split's k steps: the kt / U blocks of U steps (U = the main loop's
