@@ -920,16 +920,22 @@ SmallTile small_plan(int64_t m, int64_t n, int64_t k) {
     }
   }
   // Grids of 64 x 128 tiles short of 192 workgroups: 64 x 64 tiles (four weight
-  // and activation register stages) where they make at least 128, else 32 x 64. A
+  // and activation register stages) where they make 128 to 256, fewer 32 x 64. A
   // workgroup's time per k step is latency, not products, so more and narrower
   // workgroups are what fills the GPU; the same bits. Weights streamed, before (64 x
   // 128) -> after: 320 x 6144 x 2048 (m x k x n) 21.4 -> 14.8 us, 320 x 4096 x 2560
-  // 16.1 -> 10.9, 576 x 6144 x 2048 21.2 -> 20.1, 320 x 2048 x 2048 7.8 -> 5.8; 32 x 64
-  // against 64 x 64: 176 x 6144 x 2048 10.8 against 13.7, 64 x 4096 x 4096 9.6 against
-  // 11.8, and the other way round at 320 x 6144 x 2048, 15.5 against 14.8.
-  if (n % 128 == 0 && (m + 63) / 64 * (n / 128) < 192)
-    return (m + 63) / 64 * (n / 64) >= 128 ? SmallTile{64, 16} : SmallTile{32, 16};
-  return t;
+  // 16.1 -> 10.9, 320 x 2048 x 2048 7.8 -> 5.8; 32 x 64 against 64 x 64: 176 x 6144 x
+  // 2048 10.8 against 13.7, 64 x 4096 x 4096 9.6 against 11.8, and the other way round
+  // at 320 x 6144 x 2048, 15.5 against 14.8. Past 256 the second round of 64 x 64 tiles
+  // costs more than the wider tile: 64 x 128 against 64 x 64 at 64 x 2560 x 19456 16.4
+  // against 18.8 us, 176 x 2560 x 6144 10.7 against 12.0, 176 x 4096 x 6144 16.6 against
+  // 18.4, 320 x 4096 x 4096 13.5 against 14.8, 700 x 6144 x 2048 17.0 against 19.0,
+  // except where its grid is not a whole number per XCD and so runs without their order
+  // (400 x 4096 x 2560, 140 tiles: 15.7 against 13.7; 576, 180: 18.1 against 13.9).
+  const int64_t t128 = (m + 63) / 64 * (n / 128);
+  if (n % 128 || t128 >= 192) return t;
+  if (2 * t128 > 256 && t128 % kXcds == 0) return SmallTile{64, 32};
+  return 2 * t128 >= 128 ? SmallTile{64, 16} : SmallTile{32, 16};
 }
 
 template <int BM, int CW>

@@ -445,11 +445,13 @@ def test_gemm_fp8_pk_unsplit_row_tiles(gpu, m, n, k):
 
 
 # grids of 64 x 128 tiles short of the GPU: 32 x 64 tiles (5 .. 65 rows, one row tile
-# and its edges; the smallest n and k) and 64 x 64 tiles from 128 of them up (ragged
-# last row tile; an odd number of unrolled k blocks); 176 x 6144 x 4096 runs unsplit
+# and its edges; the smallest n and k), 64 x 64 tiles from 128 of them up (ragged last
+# row tile; an odd number of unrolled k blocks) and, past 256 of those, 64 x 128 tiles
+# (a whole number per XCD: 64 x 19456, 576 x 2048, 176 x 6144) or 64 x 64 (400 x 2560)
 @pytest.mark.parametrize("m,n,k", [(5, 128, 512), (31, 128, 1536), (32, 2048, 2048), (33, 2048, 512), (65, 1024, 1024),
                                    (300, 1024, 512), (320, 2048, 6144), (257, 2048, 1536), (576, 2048, 2048),
-                                   (320, 2560, 4096), (176, 6144, 4096)])
+                                   (320, 2560, 4096), (176, 6144, 4096), (64, 19456, 512), (400, 2560, 1536),
+                                   (512, 2048, 512)])
 @pytest.mark.parametrize("rows", [True, False])
 def test_gemm_fp8_pk_narrow_tiles(gpu, m, n, k, rows):
     """The narrow packed tiles: bit for bit ff_gemm_fp8 on the row-major codes, with
