@@ -129,8 +129,16 @@ ROWS_MAX_CODES = 49152  # FF_LINEAR_FP8_ROWS_MAX
 def rows_fit(op, m):
     """Whether ``m`` rows of ``op`` run as one launch (``linear_rows``): the op keeps
     only its packed codes, so that the single-row kernel is the one its product
-    takes anyway, and the rows' codes fit the kernel's LDS."""
-    return m <= 4 and m * op.weight.shape[1] <= ROWS_MAX_CODES and isinstance(op.weight, PackedCodes) and m > 0
+    takes anyway, and the rows' codes fit the kernel's LDS. Every 16 output columns'
+    workgroup quantises all the rows, and per-token rows one after the other (a
+    maximum each), so two to four of them only pay up to 32768 columns among them: in
+    graphs, two launches against one, 4 x 8192 x 5120 (m x k x n) 30.5 against 29.2 us,
+    4 x 4096 x 6144 18.3 against 18.1; 4 x 2560 x 19456 24.5 against 27.9, 4 x 5120 x
+    51200 90 against 102. One row, 1 x 5120 x 51200, 56.5 against 54.8; static rows
+    need no maximum and gain throughout, 4 x 5120 x 51200 87.6 against 82.8."""
+    n, k = op.weight.shape
+    return (0 < m <= 4 and m * k <= ROWS_MAX_CODES and isinstance(op.weight, PackedCodes) and
+            (m == 1 or m * n <= 32768 or isinstance(op, StaticFP8Linear)))
 
 
 def linear_rows(op, x, y):

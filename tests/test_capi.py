@@ -138,3 +138,23 @@ def test_fp8_pk_split_plan(lib_path, m, n, k, bm, splits):
     from fastforward_amd.linear import gemm_pk_workspace
     need = gemm_pk_workspace(m, n, k)
     assert need == ((m + bm - 1) // bm * (n // 256) * splits * bm * 256 * 4 if splits > 1 else 0)
+
+
+def test_rows_in_one_launch_where_they_gain():
+    """``rows_fit``: one row always, two to four per-token rows up to 32768 columns among
+    them, static-scale rows whatever the columns; never past the kernel's LDS nor where
+    the row-major codes are kept."""
+    import torch
+    from fastforward_amd.linear import FP8Linear, PackedCodes, StaticFP8Linear, rows_fit
+
+    def op(cls, n, k, packed=True):
+        o = object.__new__(cls)
+        o.weight = PackedCodes(torch.empty(0), (n, k)) if packed else torch.empty((n, k), device="meta")
+        return o
+    for m, n, k, dynamic, static in ((1, 51200, 5120, True, True), (4, 8192, 4096, True, True),
+                                     (4, 8208, 4096, False, True), (2, 19456, 2560, False, True),
+                                     (2, 12288, 4096, True, True), (2, 5120, 25600, False, False),
+                                     (5, 128, 512, False, False), (0, 128, 512, False, False)):
+        assert rows_fit(op(FP8Linear, n, k), m) is dynamic, (m, n, k)
+        assert rows_fit(op(StaticFP8Linear, n, k), m) is static, (m, n, k)
+        assert not rows_fit(op(FP8Linear, n, k, False), m)
