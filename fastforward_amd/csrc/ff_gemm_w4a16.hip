@@ -1031,12 +1031,16 @@ bool w4pk_gemv_fits(int64_t m, int64_t n, int64_t k, int64_t group) {
 //
 // BM: a wave dequantises its weights once for its BM rows, so tall tiles spend the
 // least dequantisation per product, but the rows past m are wasted. A step costs
-// about BM + 16 rows' time down to 96 rows, where the dequantisation takes as long
-// as the MFMAs. What the choice gives over 144 rows throughout (weights streamed):
+// about BM + 112 rows' time (one round of 96, 112 and 128 rows against 144: 0.80,
+// 0.89 and 0.95), 17.9 ns per row and 256 k, and a partial sum written and read 1e-6 us.
+// What the choice gives over 144 rows throughout (weights streamed):
 // gate/up of 176 tokens 2560 -> 2 x 9728 (group 32) 46.6 -> 37.7 us, 4096 -> 2 x
 // 12288 91.8 -> 73.7; 320 tokens 2048 -> 2 x 6144 49.4 -> 39.6; down of 176 tokens
-// 12288 -> 4096 42.7 -> 34.0; 576 tokens keep 144.
+// 12288 -> 4096 42.7 -> 34.0; 576 tokens keep 144, and so do 400 of 5120 -> 2 x 25600
+// (three rounds, 235 us, of 96 rows four, 251) and 130 of 25600 -> 5120 (59.5 us; 96
+// rows 62.3).
 constexpr int kW4BM = 144;
+constexpr int kW4Step = 112;  // of a step's cost, in rows
 constexpr int kW4Rows[4] = {144, 128, 112, 96};
 
 struct W4PkPlan {
@@ -1075,7 +1079,8 @@ W4PkPlan w4pk_plan(int64_t m, int64_t n, int64_t k, int64_t group) {
     if (const int f = ff_tuning(FF_TUNE_W4A16_SPLITS)) s = f;
     else if (tiles < 192) s = 256 / tiles;
     s = std::max<int64_t>(1, std::min<int64_t>({s, 8, pairs}));
-    const int64_t cost = (tiles * s + 255) / 256 * ((pairs + s - 1) / s) * (bm + 16);
+    const int64_t cost = (tiles * s + 255) / 256 * ((pairs + s - 1) / s) * (bm + kW4Step) * 179 +
+                         (s > 1 ? s * m * n / 100 : 0);
     if (p.cw == 0 || cost < best) {
       p.cw = 64;
       p.splits = (int)s;
@@ -1102,11 +1107,11 @@ int64_t w4pk_workspace(int64_t m, int64_t n, int64_t k, int64_t group) {
 }
 
 // Row-tile height of the packed SwiGLU GEMM: the fewest rounds of 256 workgroups x
-// (BM + 16) rows per CU, the tallest among equals. With 96-channel wave tiles 160
+// (BM + kW4Step) rows per CU, the tallest among equals. With 96-channel wave tiles 160
 // rows are the most the accumulators fit (240 of 256 AGPRs): the 8B gate/up at
 // 577..640 and 1153..1280 tokens keeps its rounds with them.
 int w4_swiglu_bm(int64_t m, int64_t tiles_n, int cw) {
-  const auto cost = [&](int bm) { return ((m + bm - 1) / bm * tiles_n + 255) / 256 * (bm + 16); };
+  const auto cost = [&](int bm) { return ((m + bm - 1) / bm * tiles_n + 255) / 256 * (bm + kW4Step); };
   int best = kW4BM;
   for (const int bm : kW4Rows)
     if (cost(bm) < cost(best)) best = bm;

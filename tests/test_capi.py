@@ -158,3 +158,19 @@ def test_rows_in_one_launch_where_they_gain():
         assert rows_fit(op(FP8Linear, n, k), m) is dynamic, (m, n, k)
         assert rows_fit(op(StaticFP8Linear, n, k), m) is static, (m, n, k)
         assert not rows_fit(op(FP8Linear, n, k, False), m)
+
+
+# (m, n, k, row tile, splits): 144 rows where a lower tile would take another round or more
+# k steps (130 x 5120 x 25600, 400 x 4096 x 12288), 96 where it does not and where a second
+# row tile only fills the GPU (100 and 130 x 4096 x 2048), unsplit grids (0)
+@pytest.mark.parametrize("m,n,k,bm,splits", [(130, 5120, 25600, 144, 8), (400, 4096, 12288, 144, 5),
+                                             (500, 4096, 4096, 128, 4), (100, 4096, 2048, 96, 8),
+                                             (130, 4096, 2048, 96, 8), (700, 4096, 2048, 96, 2),
+                                             (576, 4096, 12288, 144, 4), (1024, 10240, 5120, 96, 0)])
+def test_w4a16_pk_plan(lib_path, m, n, k, bm, splits):
+    """Row tile and k splits of the packed W4A16 product, from the workspace it asks for."""
+    from fastforward_amd import _lib
+    _lib.load()
+    need = ctypes.c_int64(-1)
+    _lib.call("ff_gemm_w4a16_pk_workspace", m, n, k, 128, ctypes.byref(need))
+    assert need.value == -(-m // bm) * bm * n * splits * 4

@@ -64,7 +64,8 @@ def _pk_plan(m, n, k, forced=0):
     for bm in (144, 128, 112, 96):
         tiles = -(-m // bm) * (n // 256)
         s = max(1, min(forced or (1 if tiles >= 192 else 256 // tiles), 8, pairs))
-        plans.append((-(-tiles * s // 256) * -(-pairs // s) * (bm + 16), bm, s))
+        partials = s * m * n // 100 if s > 1 else 0
+        plans.append((-(-tiles * s // 256) * -(-pairs // s) * (bm + 112) * 179 + partials, bm, s))
     _, bm, s = min(plans, key=lambda p: p[0])    # the first, tallest, of equals
     return bm, s
 
@@ -73,7 +74,7 @@ def _swiglu_rows(m, i):
     """Row-tile height of the packed SwiGLU product (mirrors w4_swiglu_bm)."""
     cw = 96 if i % 192 == 0 else 64
     return min((144, 128, 112, 96) + ((160,) if cw == 96 else ()),
-               key=lambda bm: -(-(-(-m // bm) * (i // (2 * cw))) // 256) * (bm + 16))
+               key=lambda bm: -(-(-(-m // bm) * (i // (2 * cw))) // 256) * (bm + 112))
 
 
 def test_pack_weight_int4_layout(gpu):
